@@ -13,7 +13,7 @@
  * Input features per voxel: relative dose D / D_ref (D_ref = mean dose over
  * voxels of material != 0), density (g/cm3), a material embedding scalar
  * (mass attenuation at 60 keV over water's), relative standard error.
- * Activations and weights are BF16 in channel-last layout; every convolution
+ * Activations and weights are BF16 in matrix-operand order; every convolution
  * is an implicit GEMM on CDNA4 BF16 matrix cores with FP32 accumulation;
  * Adam keeps FP32 master weights.  Volumes must have an x extent that is a
  * multiple of 64 (callers pad).
@@ -72,7 +72,7 @@ int dxg_denoiser_apply(dxg_denoiser* d, const dxg_world* w, double* dose_mgy);
 /* Test aid (no counterpart in the reference): the body-tile list that
  * dxg_denoiser_apply runs convolution `layer` (0..17) on — the tiles within
  * 19 - layer voxels of material != 0 — built on the device (host = 0) or by
- * the host scan (host = 1).  With row pairs (the default) an entry is
+ * the host scan (host = 1).  An entry is
  * pair << 2 | rows to store, pair = (z * ceil(ny / 2) + y / 2) * nx_tiles + x / 64,
  * ascending.  Up to cap entries go to out; *count receives the length. */
 int dxg_denoiser_debug_tiles(dxg_denoiser* d, const dxg_world* w, int host, int layer, int32_t* out, uint64_t cap,

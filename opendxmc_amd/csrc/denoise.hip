@@ -2,8 +2,8 @@
 // FP32 accumulation, hand-written backward pass and Adam (C-ABI in
 // include/dxmc_denoise.h).
 //
-// Tensors are channel-last BF16 with 32 channels: voxel v = ((n*D + z)*H + y)*W + x
-// occupies 64 bytes.  Every layer is a 3x3x3 convolution 32 -> 32 (the input
+// Tensors are BF16 with 32 channels in tiles of 64 voxels along x, each tile laid
+// out in matrix-operand order (chunkAt).  Every layer is a 3x3x3 convolution 32 -> 32 (the input
 // features and the one-channel output are zero padded to 32), so one kernel
 // serves all of them.
 //
@@ -15,9 +15,9 @@
 // Convolution (forward, and input gradient with flipped transposed weights):
 // A = weights (16 output channels x 32 input channels of one tap), B = 32
 // input channels x 16 voxels along x.  A wavefront owns 64 consecutive voxels
-// of one row and both output-channel halves: per tap 2 weight fragments from
-// LDS, 4 activation fragments (16 B per lane, coalesced 1 KB per instruction)
-// from memory, 8 MFMAs; 27 taps accumulate in 32 FP32 registers.
+// of two rows and both output-channel halves: per tap and row 2 weight
+// fragments from LDS, 4 activation fragments (each one contiguous kilobyte of
+// memory), 8 MFMAs; 27 taps accumulate in 64 FP32 registers.
 //
 // Weight gradient: dW[co][tap][ci] = sum_v g[v][co] x[v+off(tap)][ci] reduces
 // over voxels, so K runs over 32 voxels along x.  A work-group transposes one
@@ -99,11 +99,35 @@ __device__ inline bf16x8 asOperand(u32x4 v) { return __builtin_bit_cast(bf16x8, 
 
 __device__ inline u32x4 load16(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
 
-// A row of 64 voxels x 32 channels of zeros with one voxel of zeros on each
-// side (never written): the convolution's stand-in for input rows and halo
-// voxels outside the volume.  Kernels get the address of its voxel 0 (one
-// voxel in), so the halo voxels -1 and 64 of the zero row are zeros too.
-__device__ __align__(256) uint16_t kZeroRow[66 * 32];
+// Activation layout: a row's x extent in tiles of 64 voxels, 4 KB each.  Voxel
+// 4 n + j of a tile is voxel n of its phase j; the eight-channel chunk q of the
+// 16 voxels of a phase is contiguous: [phase j][chunk q][voxel n][8 channels].
+// A matrix operand of one phase (16 voxels x 32 channels, lane 16 q + n holding
+// chunk q of voxel n) is then one contiguous kilobyte read in lane order.
+constexpr int kTile = 64 * kC;          // values of a tile
+constexpr int kPhase = 16 * kC;         // ... of a phase
+constexpr int kChunk = 16 * 8;          // ... of a phase's channel chunk
+
+// Offset of channel chunk q of voxel x of a row that starts at voxel row0.
+__host__ __device__ inline size_t chunkAt(size_t row0, int x, int q)
+{
+    return (row0 + (x & ~63)) * kC + (x & 3) * kPhase + q * kChunk + ((x & 63) >> 2) * 8;
+}
+
+// Weight layout of one layer: the matrix operand of (tap, output channel half)
+// is one contiguous kilobyte, lane 16 q + r holding the input channels 8 q ..
+// 8 q + 7 of output channel 16 half + r.
+__host__ __device__ inline int weightAt(int tap, int co, int ci)
+{
+    return (((tap * 2 + (co >> 4)) * 4 + (ci >> 3)) * 16 + (co & 15)) * 8 + (ci & 7);
+}
+
+// A tile of zeros with zeros on both sides (never written): the convolution's
+// stand-in for input rows and halo voxels outside the volume.  Kernels get the
+// address of its voxel 0; the halo voxels x0 - 1 and x0 + 64 of a row lie up to
+// kHaloReach values before and after a tile.
+constexpr int kHaloReach = 512;
+__device__ __align__(256) uint16_t kZeroRow[kTile + 2 * kHaloReach];
 
 // ---------------------------------------------------------------- kernels
 
@@ -123,7 +147,7 @@ __global__ __launch_bounds__(64) void mfma_probe_kernel(const float* a, const fl
 
 struct ConvArgs {
     const uint16_t* x;       // input tensor
-    const uint16_t* w;       // [27][32 out][32 in] BF16
+    const uint16_t* w;       // BF16, weightAt
     const float* bias;       // 32 or null
     const uint16_t* res;     // residual added before the activation, or null (may alias y)
     const uint16_t* gate;    // output multiplied by (gate > 0), or null
@@ -134,19 +158,14 @@ struct ConvArgs {
     int nb, nz, ny, nx;
     int wave_tiles;          // tiles (or row pairs) to compute: nb*nz*ny*(nx/64), or the length of `tiles`
     int chunk;               // work-group tiles (4 wave tiles) per work-group
-    const int* tiles;        // null: every tile; else the (ascending) tile indices to compute (pair entries: conv3d_pair_kernel)
+    const int* tiles;        // null: every tile; else the (ascending) tile indices to compute (pair entries: conv3d_rows_kernel)
     int in4;                 // the network's first layer: x is the 4-channel compact input (8 bytes per voxel), conv3d_first_kernel
     const uint16_t* zrow;    // voxel 0 of kZeroRow on the device (set by launchConv)
 };
 
-// Weight fragment (tap, out channel co, 16-B chunk q) lives at chunk
-// position q ^ ((co >> 2) & 3) of its 64-B row: 16 lanes reading 16
-// consecutive rows then touch 16 distinct bank groups.
-__device__ inline int wSlot(int tap, int co, int q) { return (tap * 32 + co) * 4 + (q ^ ((co >> 2) & 3)); }
-
 // DPP row moves (16-lane rows) on the four dwords of an operand fragment;
 // lanes whose source falls outside their row keep `old`.
-constexpr int kRowShl1 = 0x101, kRowShl15 = 0x10F, kRowShr1 = 0x111, kRowShr15 = 0x11F;
+constexpr int kRowShl1 = 0x101, kRowShr1 = 0x111;
 
 template <int CTRL>
 __device__ inline u32x4 dpp4(u32x4 old, u32x4 src)
@@ -176,246 +195,31 @@ constexpr int kConvRows = DXG_CONV_ROWS;
 #define DXG_CONV_RING 3
 #endif
 constexpr int kConvRing = DXG_CONV_RING;
-// One wavefront tile: 64 voxels of one x row.
-struct Tile {
+// A row-pair tile (64 voxels along x) with what its input rows need: the
+// address of voxel x0 of row y, plane z; bit q of `rows` set when input row q
+// lies inside the volume; whether the halo voxels x0 - 1 and x0 + 64 exist.
+struct RowsTile {
     int x0, y, z, n;
     bool valid;
-};
-// A row-pair tile with what its input rows need: the address of voxel x0 of
-// row y, plane z; bit q of `rows` set when input row q lies inside the
-// volume; whether the halo voxels x0 - 1 and x0 + 64 exist.
-struct RowsTile : Tile {
     const uint16_t* own;
     uint32_t rows;
     bool left, right;
 };
 
-template <bool SHIFT>
-__global__ __launch_bounds__(64 * kConvWaves) void conv3d_kernel(ConvArgs a)
-{
-    __shared__ u32x4 wl[kTaps * 32 * 4];   // 55,296 B
-    const int tid = threadIdx.x;
-    for (int i = tid; i < kTaps * 32 * 4; i += 64 * kConvWaves) {
-        const int row = i >> 2;
-        wl[wSlot(row >> 5, row & 31, i & 3)] = reinterpret_cast<const u32x4*>(a.w)[i];
-    }
-    __syncthreads();
-
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lr = lane & 15, lq = lane >> 4;
-    float bias[2][4];
-    for (int m = 0; m < 2; ++m)
-        for (int i = 0; i < 4; ++i)
-            bias[m][i] = a.bias ? a.bias[16 * m + 4 * lq + i] : 0.0f;
-
-    // XCD-aware order: consecutive work-group ids alternate between the 8
-    // XCDs, so map them to contiguous slabs of rows per XCD.
-    const int g = gridDim.x;
-    const int logical = (blockIdx.x & 7) * (g >> 3) + (blockIdx.x >> 3);
-    const int wg_tiles = (a.wave_tiles + kConvWaves - 1) / kConvWaves;
-    const int begin = logical * a.chunk;
-    const int end = min(begin + a.chunk, wg_tiles);
-    const int nxs = a.nx >> 6;
-    auto tileAt = [&](int wt) {
-        Tile tc { 0, 0, 0, 0, false };
-        const int k = wt * kConvWaves + wave;
-        if (wt < end && k < a.wave_tiles) {
-            const int t = a.tiles ? a.tiles[k] : k;
-            int r = t / nxs;
-            tc.x0 = (t - r * nxs) * 64;
-            tc.y = r % a.ny;
-            r /= a.ny;
-            tc.z = r % a.nz;
-            tc.n = r / a.nz;
-            tc.valid = true;
-        }
-        return tc;
-    };
-
-    // Input rows (SHIFT): the nine (dz, dy) rows of a tile in turn, each
-    // loaded once.  Tile j, lane n holds voxel x0 + 4n + j (the four tiles
-    // interleave), so the x-neighbour operands of tiles 1-3 / 0-2 are simply
-    // the neighbouring tile's registers; only tile 0 at dx = -1 and tile 3 at
-    // dx = +1 take their voxel from the next lane of the same 16-lane row (one
-    // DPP move per register), with the halo voxel x0 - 1 / x0 + 64 in the lane
-    // that falls off the row.
-    // Rows stream through a ring of three buffers two rows ahead of the
-    // MFMAs, across tiles: the next tile's first two rows load during this
-    // tile's last two, so a tile does not start by waiting for its first row.
-    // Nine rows per tile keep row q of every tile in buffer q % 3.  Every row
-    // issues the same six loads (four operand chunks and the two halo voxels)
-    // whatever the position: rows outside the volume, halo voxels beyond its x
-    // ends and rows of a missing next tile read a clamped in-range address and
-    // are dropped afterwards (wave-uniform tests).  The fixed count lets the
-    // wait before a row's MFMAs cover that row only.
-    constexpr int kRing = 3;
-    const u32x4 zero = { 0, 0, 0, 0 };
-    u32x4 buf[kRing][4], lbuf[kRing], rbuf[kRing];
-    bool have[kRing] = { false, false, false };
-    auto loadRow = [&](const Tile& tc, int q, int b) {
-        const int zz = tc.z + q / 3 - 1, yy = tc.y + q % 3 - 1;
-        have[b] = tc.valid && static_cast<unsigned>(zz) < static_cast<unsigned>(a.nz) && static_cast<unsigned>(yy) < static_cast<unsigned>(a.ny);
-        const int zc = min(max(zz, 0), a.nz - 1), yc = min(max(yy, 0), a.ny - 1);
-        const size_t rowb = (static_cast<size_t>(tc.n * a.nz + zc) * a.ny + yc) * a.nx;
-        const uint16_t* base = a.x + (rowb + tc.x0 + 4 * lr) * kC + 8 * lq;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            buf[b][j] = load16(base + j * kC);
-        lbuf[b] = load16(a.x + (rowb + max(tc.x0 - 1, 0)) * kC + 8 * lq);
-        rbuf[b] = load16(a.x + (rowb + min(tc.x0 + 64, a.nx - 1)) * kC + 8 * lq);
-    };
-
-    Tile cur = tileAt(begin);
-    if (SHIFT && cur.valid) {
-        loadRow(cur, 0, 0);
-        loadRow(cur, 1, 1);
-    }
-    for (int wt = begin; cur.valid; ++wt) {
-        const Tile nxt = tileAt(wt + 1);
-        const int x0 = cur.x0, y = cur.y, z = cur.z, n = cur.n;
-
-        f32x4 acc[2][4];
-        for (int m = 0; m < 2; ++m)
-            for (int j = 0; j < 4; ++j)
-                acc[m][j] = f32x4 { 0, 0, 0, 0 };
-
-        // The epilogue's residual (or gate) values, loaded before the MFMAs
-        // so that their latency hides behind them; loaded after them, each
-        // store's possible alias with the next load serialised the waits.
-        // The residual may alias the output: each tile reads and writes only
-        // its own voxels.
-        const size_t orow = (static_cast<size_t>(n * a.nz + z) * a.ny + y) * a.nx;
-        u32x2 side[4][2];
-        const uint16_t* side_src = a.res ? a.res : a.gate;
-        if (side_src) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const size_t v = orow + x0 + (SHIFT ? 4 * lr + j : 16 * j + lr);
-#pragma unroll
-                for (int m = 0; m < 2; ++m)
-                    side[j][m] = *reinterpret_cast<const u32x2*>(side_src + v * kC + 16 * m + 4 * lq);
-            }
-        }
-
-        if (SHIFT) {
-#pragma unroll
-            for (int q = 0; q < 9; ++q) {
-                const int b = q % kRing;
-                if (q + 2 < 9)
-                    loadRow(cur, q + 2, (q + 2) % kRing);
-                else
-                    loadRow(nxt, q + 2 - 9, (q + 2) % kRing);
-                if (!have[b])
-                    continue;
-                const u32x4(&c)[4] = buf[b];
-#pragma unroll
-                for (int dx = -1; dx <= 1; ++dx) {
-                    bf16x8 bop[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        if (dx == 0)
-                            bop[j] = asOperand(c[j]);
-                        else if (dx < 0)
-                            bop[j] = asOperand(j > 0 ? c[j - 1] : dpp4<kRowShr1>(x0 > 0 ? lbuf[b] : zero, c[3]));   // lane n <- lane n-1
-                        else
-                            bop[j] = asOperand(j < 3 ? c[j + 1] : dpp4<kRowShl1>(x0 + 64 < a.nx ? rbuf[b] : zero, c[0]));   // lane n <- lane n+1
-                    }
-                    const int tap = q * 3 + dx + 1;
-                    bf16x8 aop[2];
-#pragma unroll
-                    for (int m = 0; m < 2; ++m)
-                        aop[m] = asOperand(wl[wSlot(tap, 16 * m + lr, lq)]);
-#pragma unroll
-                    for (int m = 0; m < 2; ++m)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aop[m], bop[j], acc[m][j], 0, 0, 0);
-                }
-            }
-        }
-        for (int dz = -1; dz <= 1 && !SHIFT; ++dz) {
-            const int zz = z + dz;
-            if (static_cast<unsigned>(zz) >= static_cast<unsigned>(a.nz))
-                continue;
-            for (int dy = -1; dy <= 1; ++dy) {
-                const int yy = y + dy;
-                if (static_cast<unsigned>(yy) >= static_cast<unsigned>(a.ny))
-                    continue;
-                const size_t rowb = (static_cast<size_t>(n * a.nz + zz) * a.ny + yy) * a.nx;
-                const int tapb = (dz + 1) * 9 + (dy + 1) * 3;
-#pragma unroll
-                for (int dx = -1; dx <= 1; ++dx) {
-                    bf16x8 bop[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int xx = x0 + 16 * j + lr + dx;
-                        u32x4 v = { 0, 0, 0, 0 };
-                        if (static_cast<unsigned>(xx) < static_cast<unsigned>(a.nx))
-                            v = load16(a.x + (rowb + xx) * kC + 8 * lq);
-                        bop[j] = asOperand(v);
-                    }
-                    const int tap = tapb + dx + 1;
-                    bf16x8 aop[2];
-#pragma unroll
-                    for (int m = 0; m < 2; ++m)
-                        aop[m] = asOperand(wl[wSlot(tap, 16 * m + lr, lq)]);
-#pragma unroll
-                    for (int m = 0; m < 2; ++m)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aop[m], bop[j], acc[m][j], 0, 0, 0);
-                }
-            }
-        }
-
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const size_t v = orow + x0 + (SHIFT ? 4 * lr + j : 16 * j + lr);
-#pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                const int co0 = 16 * m + 4 * lq;
-                float o[4];
-                for (int i = 0; i < 4; ++i)
-                    o[i] = acc[m][j][i] + bias[m][i];
-                if (a.res) {
-                    const u32x2 rv = side[j][m];
-                    o[0] += fromBf16(rv[0] & 0xffffu);
-                    o[1] += fromBf16(rv[0] >> 16);
-                    o[2] += fromBf16(rv[1] & 0xffffu);
-                    o[3] += fromBf16(rv[1] >> 16);
-                }
-                if (a.relu)
-                    for (int i = 0; i < 4; ++i)
-                        o[i] = fmaxf(o[i], 0.0f);
-                if (a.gate) {
-                    const u32x2 gv = a.res ? *reinterpret_cast<const u32x2*>(a.gate + v * kC + co0) : side[j][m];
-                    const uint32_t h[4] = { gv[0] & 0xffffu, gv[0] >> 16, gv[1] & 0xffffu, gv[1] >> 16 };
-                    for (int i = 0; i < 4; ++i)
-                        if (h[i] == 0 || (h[i] & 0x8000u))
-                            o[i] = 0.0f;
-                }
-                if (a.y)
-                    *reinterpret_cast<u32x2*>(a.y + v * kC + co0) = u32x2 { pack2(o[0], o[1]), pack2(o[2], o[3]) };
-                if (a.y32) {
-                    if (a.y32_channels == kC)
-                        *reinterpret_cast<f32x4*>(a.y32 + v * kC + co0) = f32x4 { o[0], o[1], o[2], o[3] };
-                    else if (co0 == 0)
-                        a.y32[v] = o[0];
-                }
-            }
-        }
-        cur = nxt;
-    }
-}
-
-
 // Row-pair convolution: a wavefront computes output rows y and y + 1 (64
 // voxels each, same x range) together.  Their 3x3 input-row neighbourhoods
 // overlap in six of nine rows per pair of rows: the pair streams the twelve
 // rows (dz, y - 1 .. y + 2) once and applies each to both outputs (rows y and
-// y + 1 feed six taps), so it loads 12 rows where two single-row tiles load
-// 18; the input loads, not the MFMAs or the weight reads, bound the
-// single-row kernel.  Same operand layout and ring as conv3d_kernel<true>;
-// twelve rows per pair keep row q of every pair in buffer q % 3.
+// y + 1 feed six taps), so it loads 12 rows where two single rows load 18.
+// Tile j of a row holds its phase j (voxels x0 + 4 n + j, lane n), so the
+// x-neighbour operands of phases 1-3 / 0-2 are simply the neighbouring phase's
+// registers; only phase 0 at dx = -1 and phase 3 at dx = +1 take their voxel
+// from the next lane of the same 16-lane row (one DPP move per register), with
+// the halo voxel x0 - 1 / x0 + 64 in the lane that falls off the row.
+// Rows stream through a ring of three buffers two rows ahead of the MFMAs and
+// across tiles; every row issues the same six loads whatever the position, so
+// that the wait before a row's MFMAs covers that row only.  Twelve rows per
+// pair keep row q of every pair in buffer q % 3.
 // Entries of a.tiles (when given) are pair * 4 + mask: bit 0 stores row y,
 // bit 1 row y + 1 (a pair index counts (n, z, y / 2, x / 64) like a tile
 // index with ceil(ny / 2) rows); without a list every pair is computed and
@@ -447,10 +251,8 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
     constexpr int kHalves = EPI == kEpiY32 ? 1 : 2;
     __shared__ u32x4 wl[kTaps * 32 * 4];   // 55,296 B
     const int tid = threadIdx.x;
-    for (int i = tid; i < kTaps * 32 * 4; i += 64 * kConvWaves) {
-        const int row = i >> 2;
-        wl[wSlot(row >> 5, row & 31, i & 3)] = reinterpret_cast<const u32x4*>(a.w)[i];
-    }
+    for (int i = tid; i < kTaps * 32 * 4; i += 64 * kConvWaves)
+        wl[i] = reinterpret_cast<const u32x4*>(a.w)[i];
     __syncthreads();
 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lr = lane & 15, lq = lane >> 4;
@@ -519,18 +321,20 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
     // read from the zero row, so no address is clamped and the shifted
     // operands need no selects; a skipped row's halo voxels are the zero
     // row's padding.
-    const uint32_t lane_off = 4 * lr * kC + 8 * lq;
+    const uint32_t lane_off = 8 * lane;
+    // the lane's four output channels 4 lq .. of voxel lr of a phase, half 0
+    const uint32_t out_off = (lq >> 1) * kChunk + lr * 8 + (lq & 1) * 4;
     auto loadRow = [&](const RowsTile& tc, int q, int b) {
         const int dz = q / (R + 2) - 1, dy = q % (R + 2) - 1;
         have[b] = (tc.rows >> q) & 1u;
         const uint16_t* row = have[b] ? tc.own + dz * plane_stride + dy * row_stride : zrow;
-        const uint16_t* left = tc.left ? row - kC : zrow;
-        const uint16_t* right = tc.right ? row + 64 * kC : zrow;
+        const uint16_t* left = tc.left ? row - kTile + 3 * kPhase + 15 * 8 : zrow;   // voxel 15 of phase 3 of the tile before
+        const uint16_t* right = tc.right ? row + kTile : zrow;                        // voxel 0 of phase 0 of the tile after
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            buf[b][j] = load16(row + lane_off + j * kC);
-        lbuf[b] = load16(left + 8 * lq);
-        rbuf[b] = load16(right + 8 * lq);
+            buf[b][j] = load16(row + lane_off + j * kPhase);
+        lbuf[b] = load16(left + kChunk * lq);
+        rbuf[b] = load16(right + kChunk * lq);
     };
     // The weight fragments of a step (one tap, both channel halves) are read
     // from LDS one step ahead of their MFMAs.  The steps of a tile run over
@@ -551,7 +355,7 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
     bf16x8 wcur[2];
 #pragma unroll
     for (int m = 0; m < kHalves; ++m)
-        wcur[m] = asOperand(wl[wSlot(0, 16 * m + lr, lq)]);
+        wcur[m] = asOperand(wl[m * 64 + lane]);
 
     int cmask = 0;
     RowsTile cur = tileAt(begin, cmask);
@@ -581,12 +385,11 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
                 if (!((cmask >> o) & 1))
                     continue;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const size_t v = orow0 + static_cast<size_t>(o) * a.nx + x0 + 4 * lr + j;
+                for (int j = 0; j < 4; ++j)
 #pragma unroll
                     for (int m = 0; m < 2; ++m)
-                        side[o][j][m] = *reinterpret_cast<const u32x2*>(side_src + v * kC + 16 * m + 4 * lq);
-                }
+                        side[o][j][m] = *reinterpret_cast<const u32x2*>(side_src + (orow0 + static_cast<size_t>(o) * a.nx + x0) * kC + out_off
+                                                                        + j * kPhase + m * 2 * kChunk);
             }
         }
 
@@ -602,7 +405,7 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
                 const int tap_next = nextTap(q, 1, R - 1);
 #pragma unroll
                 for (int m = 0; m < kHalves; ++m)
-                    wcur[m] = asOperand(wl[wSlot(tap_next, 16 * m + lr, lq)]);
+                    wcur[m] = asOperand(wl[(tap_next * 2 + m) * 64 + lane]);
                 continue;
             }
             const int rr = q % (R + 2);   // input row y + rr - 1 of plane z + q / (R + 2) - 1
@@ -628,7 +431,7 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
                     bf16x8 wnext[2];
 #pragma unroll
                     for (int m = 0; m < kHalves; ++m)
-                        wnext[m] = asOperand(wl[wSlot(tap_next, 16 * m + lr, lq)]);
+                        wnext[m] = asOperand(wl[(tap_next * 2 + m) * 64 + lane]);
 #pragma unroll
                     for (int m = 0; m < kHalves; ++m)
 #pragma unroll
@@ -654,11 +457,12 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
                 for (int m = 0; m < kHalves; ++m) {
                     const int co0 = 16 * m + 4 * lq;
+                    const size_t at = (orow0 + static_cast<size_t>(o) * a.nx + x0) * kC + out_off + j * kPhase + m * 2 * kChunk;
                     float out[4];
                     for (int i = 0; i < 4; ++i)
                         out[i] = acc[o][m][j][i] + bias[m][i];
                     const u32x2 sv = kPrefetchSide ? side[kPrefetchSide ? o : 0][j][m]
-                                                   : ((e_res || e_gate) ? *reinterpret_cast<const u32x2*>(side_src + v * kC + co0) : u32x2 { 0, 0 });
+                                                   : ((e_res || e_gate) ? *reinterpret_cast<const u32x2*>(side_src + at) : u32x2 { 0, 0 });
                     if (e_res) {
                         const u32x2 rv = sv;
                         out[0] += fromBf16(rv[0] & 0xffffu);
@@ -670,14 +474,14 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
                         for (int i = 0; i < 4; ++i)
                             out[i] = fmaxf(out[i], 0.0f);
                     if (e_gate) {
-                        const u32x2 gv = e_res ? *reinterpret_cast<const u32x2*>(a.gate + v * kC + co0) : sv;
+                        const u32x2 gv = e_res ? *reinterpret_cast<const u32x2*>(a.gate + at) : sv;
                         const uint32_t h[4] = { gv[0] & 0xffffu, gv[0] >> 16, gv[1] & 0xffffu, gv[1] >> 16 };
                         for (int i = 0; i < 4; ++i)
                             if (h[i] == 0 || (h[i] & 0x8000u))
                                 out[i] = 0.0f;
                     }
                     if (e_y)
-                        *reinterpret_cast<u32x2*>(a.y + v * kC + co0) = u32x2 { pack2(out[0], out[1]), pack2(out[2], out[3]) };
+                        *reinterpret_cast<u32x2*>(a.y + at) = u32x2 { pack2(out[0], out[1]), pack2(out[2], out[3]) };
                     if (e_y32) {
                         if (e_y32_all)
                             *reinterpret_cast<f32x4*>(a.y32 + v * kC + co0) = f32x4 { out[0], out[1], out[2], out[3] };
@@ -740,7 +544,7 @@ __global__ __launch_bounds__(64 * kConvWaves) void conv3d_first_kernel(ConvArgs 
             for (int k = 0; k < 2; ++k) {
                 u32x2 w2 = { 0u, 0u };
                 if (tval[c][k])
-                    w2 = *reinterpret_cast<const u32x2*>(a.w + (static_cast<size_t>(8 * c + 2 * lq + k) * 32 + 16 * m + lr) * kC);
+                    w2 = *reinterpret_cast<const u32x2*>(a.w + weightAt(8 * c + 2 * lq + k, 16 * m + lr, 0));
                 v[2 * k] = w2[0];
                 v[2 * k + 1] = w2[1];
             }
@@ -819,7 +623,8 @@ __global__ __launch_bounds__(64 * kConvWaves) void conv3d_first_kernel(ConvArgs 
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const size_t v = orow + 16 * j + lr;
+                // voxel 16 j + lr of the tile, channels 16 m + 4 lq ..
+                const size_t at = orow * kC + (lr & 3) * kPhase + (lq >> 1) * kChunk + (4 * j + (lr >> 2)) * 8 + (lq & 1) * 4;
 #pragma unroll
                 for (int m = 0; m < 2; ++m) {
                     float out[4];
@@ -828,7 +633,7 @@ __global__ __launch_bounds__(64 * kConvWaves) void conv3d_first_kernel(ConvArgs 
                         if (a.relu)
                             out[i] = fmaxf(out[i], 0.0f);
                     }
-                    *reinterpret_cast<u32x2*>(a.y + v * kC + 16 * m + 4 * lq) = u32x2 { pack2(out[0], out[1]), pack2(out[2], out[3]) };
+                    *reinterpret_cast<u32x2*>(a.y + at + m * 2 * kChunk) = u32x2 { pack2(out[0], out[1]), pack2(out[2], out[3]) };
                 }
             }
         }
@@ -904,8 +709,8 @@ __global__ __launch_bounds__(256) void wgrad_kernel(WgradArgs a)
         __syncthreads();   // the previous tile is consumed
         for (int i = tid; i < 4 * 32 * 4; i += 256) {
             const int q = i & 3, vox = (i >> 2) & 31, rr = i >> 7;
-            const size_t v = (static_cast<size_t>(n * a.nz + z) * a.ny + y0 + rr) * a.nx + x0 + vox;
-            const u32x4 d = load16(a.g + v * kC + 8 * q);
+            const size_t row0 = (static_cast<size_t>(n * a.nz + z) * a.ny + y0 + rr) * a.nx;
+            const u32x4 d = load16(a.g + chunkAt(row0, x0 + vox, q));
             uint16_t* dst = gT + (rr * 32 + 8 * q) * kGtLen + vox;
             for (int e = 0; e < 4; ++e) {
                 dst[(2 * e) * kGtLen] = static_cast<uint16_t>(d[e] & 0xffffu);
@@ -919,7 +724,7 @@ __global__ __launch_bounds__(256) void wgrad_kernel(WgradArgs a)
             u32x4 d = { 0, 0, 0, 0 };
             if (static_cast<unsigned>(zz) < static_cast<unsigned>(a.nz) && static_cast<unsigned>(yy) < static_cast<unsigned>(a.ny)
                 && static_cast<unsigned>(xx) < static_cast<unsigned>(a.nx))
-                d = load16(a.x + ((static_cast<size_t>(n * a.nz + zz) * a.ny + yy) * a.nx + xx) * kC + 8 * q);
+                d = load16(a.x + chunkAt((static_cast<size_t>(n * a.nz + zz) * a.ny + yy) * a.nx, xx, q));
             uint16_t* dst = xT + (row * 32 + 8 * q) * kXtLen + vox;
             for (int e = 0; e < 4; ++e) {
                 dst[(2 * e) * kXtLen] = static_cast<uint16_t>(d[e] & 0xffffu);
@@ -1032,8 +837,8 @@ __global__ __launch_bounds__(256) void wgrad_finish_kernel(const float* sums, fl
     }
 }
 
-// FP32 master parameters -> BF16 forward weights [tap][co][ci] and input-
-// gradient weights wd[tap][co][ci] = W[ci][26 - tap][co] (flipped, transposed).
+// FP32 master parameters -> BF16 forward weights and input-gradient weights
+// wd(tap, co, ci) = W[ci][26 - tap][co] (flipped, transposed), both as weightAt.
 __global__ __launch_bounds__(256) void prep_weights_kernel(const float* params, uint16_t* wf, uint16_t* wd, int layers)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
@@ -1042,8 +847,9 @@ __global__ __launch_bounds__(256) void prep_weights_kernel(const float* params, 
     const int l = i / kLayerW, r = i - l * kLayerW;
     const int tap = r >> 10, co = (r >> 5) & 31, ci = r & 31;
     const float* p = params + static_cast<size_t>(l) * kLayerP;
-    wf[i] = toBf16(p[(co * kTaps + tap) * kC + ci]);
-    wd[i] = toBf16(p[(ci * kTaps + (kTaps - 1 - tap)) * kC + co]);
+    const int at = l * kLayerW + weightAt(tap, co, ci);
+    wf[at] = toBf16(p[(co * kTaps + tap) * kC + ci]);
+    wd[at] = toBf16(p[(ci * kTaps + (kTaps - 1 - tap)) * kC + co]);
 }
 
 __global__ __launch_bounds__(256) void adam_kernel(float* p, float* m, float* v, const float* g, int n, float lr, float b1,
@@ -1060,6 +866,17 @@ __global__ __launch_bounds__(256) void adam_kernel(float* p, float* m, float* v,
     p[i] -= lr * (mi * bc1) / (sqrtf(vi * bc2) + eps);
 }
 
+// Voxel v of a 32-channel tensor: channels 0..7 from c0, the rest zero (x
+// extents are whole tiles, so the flat voxel index gives the tile too).
+__device__ inline void storeVoxel(uint16_t* t, size_t v, u32x4 c0)
+{
+    uint16_t* p = t + chunkAt(v & ~static_cast<size_t>(63), static_cast<int>(v & 63), 0);
+    *reinterpret_cast<u32x4*>(p) = c0;
+#pragma unroll
+    for (int q = 1; q < 4; ++q)
+        *reinterpret_cast<u32x4*>(p + q * kChunk) = u32x4 { 0u, 0u, 0u, 0u };
+}
+
 // Features (4 FP32 per voxel) -> 32-channel BF16 input tensor and an FP32 copy
 // of feature 0 (the relative dose the network corrects).
 __global__ __launch_bounds__(256) void pack_features_kernel(const float* f, uint16_t* xin, uint16_t* xin4, float* feat0, size_t nv)
@@ -1068,13 +885,9 @@ __global__ __launch_bounds__(256) void pack_features_kernel(const float* f, uint
     if (v >= nv)
         return;
     const f32x4 q = *reinterpret_cast<const f32x4*>(f + 4 * v);
-    u32x4* dst = reinterpret_cast<u32x4*>(xin + v * kC);
     const u32x2 f4 = { pack2(q[0], q[1]), pack2(q[2], q[3]) };
-    dst[0] = u32x4 { f4[0], f4[1], 0u, 0u };
     *reinterpret_cast<u32x2*>(xin4 + 4 * v) = f4;
-    dst[1] = u32x4 { 0u, 0u, 0u, 0u };
-    dst[2] = u32x4 { 0u, 0u, 0u, 0u };
-    dst[3] = u32x4 { 0u, 0u, 0u, 0u };
+    storeVoxel(xin, v, u32x4 { f4[0], f4[1], 0u, 0u });
     feat0[v] = q[0];
 }
 
@@ -1091,11 +904,7 @@ __global__ __launch_bounds__(256) void loss_kernel(const float* y32, const float
         const float diff = feat0[v] + y32[v] - target[v];
         const float mk = mask[v];
         l = mk * diff * diff;
-        u32x4* dst = reinterpret_cast<u32x4*>(gout + v * kC);
-        dst[0] = u32x4 { static_cast<uint32_t>(toBf16(2.0f * mk * diff * inv_count)), 0u, 0u, 0u };
-        dst[1] = u32x4 { 0u, 0u, 0u, 0u };
-        dst[2] = u32x4 { 0u, 0u, 0u, 0u };
-        dst[3] = u32x4 { 0u, 0u, 0u, 0u };
+        storeVoxel(gout, v, u32x4 { static_cast<uint32_t>(toBf16(2.0f * mk * diff * inv_count)), 0u, 0u, 0u });
     }
     for (int off = 32; off > 0; off >>= 1)
         l += __shfl_down(l, off, 64);
@@ -1204,13 +1013,8 @@ __global__ __launch_bounds__(256) void world_features_kernel(WorldFeatArgs a)
     }
     const u32x2 f4 = { pack2(f[0], f[1]), pack2(f[2], f[3]) };
     *reinterpret_cast<u32x2*>(a.xin4 + 4 * v) = f4;
-    if (a.xin) {
-        u32x4* dst = reinterpret_cast<u32x4*>(a.xin + v * kC);
-        dst[0] = u32x4 { f4[0], f4[1], 0u, 0u };
-        dst[1] = u32x4 { 0u, 0u, 0u, 0u };
-        dst[2] = u32x4 { 0u, 0u, 0u, 0u };
-        dst[3] = u32x4 { 0u, 0u, 0u, 0u };
-    }
+    if (a.xin)
+        storeVoxel(a.xin, v, u32x4 { f4[0], f4[1], 0u, 0u });
     a.feat0[v] = f[0];
     if (a.features)
         *reinterpret_cast<f32x4*>(a.features + 4 * v) = f32x4 { f[0], f[1], f[2], f[3] };
@@ -1246,27 +1050,6 @@ int computeUnits()
 
 int roundUp8(int v) { return (v + 7) & ~7; }
 
-// Activation operands for the x-neighbour taps: moved across lanes (default)
-// or loaded again per tap (DXG_CONV_SHIFT=0).
-bool convShift()
-{
-    static const bool on = [] {
-        const char* e = std::getenv("DXG_CONV_SHIFT");
-        return !(e && e[0] == '0');
-    }();
-    return on;
-}
-
-// Row-pair convolution (conv3d_pair_kernel) unless DXG_CONV_PAIRS=0.
-bool convPairs()
-{
-    static const bool on = [] {
-        const char* e = std::getenv("DXG_CONV_PAIRS");
-        return !(e && e[0] == '0');
-    }();
-    return on;
-}
-
 // The first layer by conv3d_first_kernel (its four input channels packed
 // over the taps) unless DXG_CONV_FIRST=0.
 int convFirst()
@@ -1287,7 +1070,7 @@ struct Dims {
 // pairs on, and a plane small enough for its 32-bit offsets.
 bool firstLayerCompact(const Dims& d)
 {
-    return convFirst() && convPairs() && static_cast<long long>(d.ny + 1) * d.nx < (1ll << 27);
+    return convFirst() && static_cast<long long>(d.ny + 1) * d.nx < (1ll << 27);
 }
 
 int checkDims(const char* fn, uint64_t batch, const uint64_t* dims, Dims& d)
@@ -1320,7 +1103,7 @@ const uint16_t* zeroRow()
     void* p = nullptr;
     if (hipGetSymbolAddress(&p, HIP_SYMBOL(kZeroRow)) != hipSuccess)
         return nullptr;
-    return rows[dev] = static_cast<const uint16_t*>(p) + kC;
+    return rows[dev] = static_cast<const uint16_t*>(p) + kHaloReach;
 }
 
 hipError_t launchConv(ConvArgs a, const Dims& d, hipStream_t s)
@@ -1332,9 +1115,8 @@ hipError_t launchConv(ConvArgs a, const Dims& d, hipStream_t s)
     a.nz = d.nz;
     a.ny = d.ny;
     a.nx = d.nx;
-    const bool pairs = convPairs();
     if (!a.tiles)
-        a.wave_tiles = d.nb * d.nz * (pairs ? (d.ny + kConvRows - 1) / kConvRows : d.ny) * (d.nx / 64);
+        a.wave_tiles = d.nb * d.nz * ((d.ny + kConvRows - 1) / kConvRows) * (d.nx / 64);
     const int wg_tiles = (a.wave_tiles + kConvWaves - 1) / kConvWaves;
     const int grid = roundUp8(std::min(wg_tiles, 2 * computeUnits()));
     a.chunk = (wg_tiles + grid - 1) / grid;
@@ -1342,16 +1124,13 @@ hipError_t launchConv(ConvArgs a, const Dims& d, hipStream_t s)
     // can (its 32-bit element offsets from a row's corner stay below 2^31
     // while (ny + 1) nx < 2^27)
     if (a.in4) {
-        if (!pairs || !a.y || a.y32 || a.res || a.gate || static_cast<long long>(d.ny + 1) * d.nx >= (1ll << 27))
+        if (!a.y || a.y32 || a.res || a.gate || static_cast<long long>(d.ny + 1) * d.nx >= (1ll << 27))
             return hipErrorInvalidValue;
         hipLaunchKernelGGL(conv3d_first_kernel, dim3(grid), dim3(64 * kConvWaves), 0, s, a);
-    } else if (pairs) {
+    } else {
         void* args[] = { &a };
         (void)hipLaunchKernel(rowsKernel(a), dim3(grid), dim3(64 * kConvWaves), args, 0, s);
-    } else if (convShift())
-        hipLaunchKernelGGL(conv3d_kernel<true>, dim3(grid), dim3(64 * kConvWaves), 0, s, a);
-    else
-        hipLaunchKernelGGL(conv3d_kernel<false>, dim3(grid), dim3(64 * kConvWaves), 0, s, a);
+    }
     return hipGetLastError();
 }
 
@@ -1459,7 +1238,7 @@ void hostLayerTiles(const uint8_t* mat, int nx, int ny, int nz, int nxp, std::ve
     }
 }
 
-// The row pairs of conv3d_pair_kernel that hold the given wave tiles
+// The row pairs of conv3d_rows_kernel that hold the given wave tiles
 // (ascending tile indices of a volume with ny rows and nxt tiles per row), as
 // pair * 4 + rows to store (bit 0 row y, bit 1 row y + 1), ascending.
 std::vector<int> pairTiles(const std::vector<int>& tiles, int ny, int nxt)
@@ -1802,18 +1581,17 @@ struct dxg_denoiser {
         return DXG_OK;
     }
 
-    // The body-tile lists the convolutions take: on the device for row pairs
-    // unless DXG_DENOISE_TILES_HOST=1 (or always on the host for single rows).
+    // The body-tile lists the convolutions take: on the device unless
+    // DXG_DENOISE_TILES_HOST=1.
     int buildTiles(const dxg::WorldView& v, const Dims& dm, bool host)
     {
-        if (!host && convPairs())
+        if (!host)
             return devicePairTiles(v, dm);
         std::vector<int> t[kLayers];
         hostLayerTiles(v.material_host, v.nx, v.ny, v.nz, dm.nx, t);
         size_t most = 1;
         for (int l = 0; l < kLayers; ++l) {
-            if (convPairs())
-                t[l] = pairTiles(t[l], dm.ny, dm.nx / 64);
+            t[l] = pairTiles(t[l], dm.ny, dm.nx / 64);
             most = std::max(most, t[l].size());
         }
         tiles_stride = most;
@@ -1924,23 +1702,60 @@ struct dxg_denoiser {
 
 namespace {
 
+// Standard normals by Marsaglia's polar method in FP32 from 64-bit draws: the
+// values std::normal_distribution<float> gives here, without its two long
+// double logarithms per pair (444,000 draws: 31 ms with it, 9 ms without).
+struct Normals {
+    std::mt19937_64 rng;
+    float kept = 0.0f;
+    bool has_kept = false;
+    float uniform() { return std::min(static_cast<float>(rng()) * 0x1p-64f, 0x1.fffffep-1f); }
+    float draw()
+    {
+        if (has_kept) {
+            has_kept = false;
+            return kept;
+        }
+        float x, y, r2;
+        do {
+            x = 2.0f * uniform() - 1.0f;
+            y = 2.0f * uniform() - 1.0f;
+            r2 = x * x + y * y;
+        } while (r2 > 1.0f || r2 == 0.0f);
+        const float m = std::sqrt(-2.0f * std::log(r2) / r2);
+        kept = x * m;
+        has_kept = true;
+        return y * m;
+    }
+};
+
 void initParams(std::vector<float>& p, uint64_t seed)
 {
     p.assign(static_cast<size_t>(kLayers) * kLayerP, 0.0f);
-    std::mt19937_64 rng(seed);
+    Normals nd;
+    nd.rng.seed(seed);
     for (int l = 0; l < kLayers - 1; ++l) {
         const int ci_active = l == 0 ? DXG_DENOISE_FEATURES : kC;
         // He initialisation; the second convolution of each residual block
         // starts small so every block begins close to the identity.
         const bool second = l > 0 && (l % 2) == 0;
-        std::normal_distribution<float> nd(0.0f, (second ? 0.1f : 1.0f) * std::sqrt(2.0f / (kTaps * ci_active)));
+        const float sd = (second ? 0.1f : 1.0f) * std::sqrt(2.0f / (kTaps * ci_active));
+        nd.has_kept = false;   // a layer starts with a fresh pair
         float* w = p.data() + static_cast<size_t>(l) * kLayerP;
         for (int co = 0; co < kC; ++co)
             for (int tap = 0; tap < kTaps; ++tap)
                 for (int ci = 0; ci < ci_active; ++ci)
-                    w[(co * kTaps + tap) * kC + ci] = nd(rng);
+                    w[(co * kTaps + tap) * kC + ci] = nd.draw() * sd;
     }
     // the correction layer starts at zero: the untrained network is the identity on the log dose
+}
+
+// Where value i of a tensor in [voxel][channel] order lies on the device.
+size_t valueAt(size_t i)
+{
+    const size_t v = i / kC;
+    const int c = static_cast<int>(i % kC);
+    return chunkAt(v & ~static_cast<size_t>(63), static_cast<int>(v & 63), c >> 3) + (c & 7);
 }
 
 bool hasDevice()
@@ -2247,7 +2062,7 @@ int dxg_conv3d_probe(int mode, const float* x, const float* w, const float* bias
     const size_t nv = dm.voxels(), ts = nv * kC;
     std::vector<uint16_t> xh(ts);
     for (size_t i = 0; i < ts; ++i)
-        xh[i] = toBf16(x[i]);
+        xh[valueAt(i)] = toBf16(x[i]);
     std::vector<float> layer(kLayerP, 0.0f);
     std::copy(w, w + kLayerW, layer.begin());
     if (mode == 0 || mode == 3)
@@ -2265,7 +2080,7 @@ int dxg_conv3d_probe(int mode, const float* x, const float* w, const float* bias
     if (mode == 2) {
         std::vector<uint16_t> gh(ts);
         for (size_t i = 0; i < ts; ++i)
-            gh[i] = toBf16(bias_or_dy[i]);
+            gh[valueAt(i)] = toBf16(bias_or_dy[i]);
         HIP_TRY(dy.reserve(ts));
         HIP_TRY(hipMemcpy(dy.p, gh.data(), ts * 2, hipMemcpyHostToDevice));
         const int grid = wgradGrid(dm);
@@ -2284,11 +2099,11 @@ int dxg_conv3d_probe(int mode, const float* x, const float* w, const float* bias
             if (i % kC >= 4 && x[i] != 0.0f)
                 return fail(DXG_ERR_ARGUMENT, "dxg_conv3d_probe: mode 3 needs channels 4..31 of x to be zero");
         if (!firstLayerCompact(dm))
-            return fail(DXG_ERR_ARGUMENT, "dxg_conv3d_probe: mode 3 needs row pairs and a plane below 2^27 voxels");
+            return fail(DXG_ERR_ARGUMENT, "dxg_conv3d_probe: mode 3 needs a plane below 2^27 voxels");
         std::vector<uint16_t> x4(nv * 4);
         for (size_t v = 0; v < nv; ++v)
             for (int k = 0; k < 4; ++k)
-                x4[4 * v + k] = xh[v * kC + k];
+                x4[4 * v + k] = xh[valueAt(v * kC + k)];
         DBuf<uint16_t> yb, dx4;
         HIP_TRY(yb.reserve(ts));
         HIP_TRY(dx4.reserve(nv * 4));
@@ -2304,7 +2119,7 @@ int dxg_conv3d_probe(int mode, const float* x, const float* w, const float* bias
         std::vector<uint16_t> yh(ts);
         HIP_TRY(hipMemcpy(yh.data(), yb.p, ts * sizeof(uint16_t), hipMemcpyDeviceToHost));
         for (size_t i = 0; i < ts; ++i)
-            out[i] = fromBf16(yh[i]);
+            out[i] = fromBf16(yh[valueAt(i)]);
         return DXG_OK;
     }
     HIP_TRY(dout.reserve(ts));

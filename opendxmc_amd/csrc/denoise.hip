@@ -20,10 +20,8 @@
 // memory), 8 MFMAs; 27 taps accumulate in 64 FP32 registers.
 //
 // Weight gradient: dW[co][tap][ci] = sum_v g[v][co] x[v+off(tap)][ci] reduces
-// over voxels, so K runs over 32 voxels along x.  A work-group transposes one
-// 4-row x 32-voxel tile of g and its 18-row halo of x into channel-major LDS;
-// each wavefront keeps the partial sums of 7 taps in registers and reads the
-// x-shifted operand with two aligned 16-B reads and a byte funnel shift.
+// over voxels, so K runs over 32 voxels along x.  Rows of g and x pass through
+// LDS and are read transposed; each wavefront keeps the sums of nine taps.
 #include "dxmc_denoise.h"
 
 #include "device.hpp"
@@ -39,6 +37,7 @@
 #include <mutex>
 #include <random>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -54,8 +53,6 @@ constexpr int kLayerW = kC * kTaps * kC;             // 27648 weights per layer
 constexpr int kLayerP = kLayerW + kC;                // + 32 biases
 constexpr int kLayers = DXG_DENOISE_LAYERS;          // 18
 constexpr int kBlocks = (kLayers - 2) / 2;           // 8 residual blocks
-constexpr int kXtLen = 56;                           // halo row length in LDS (112 B: conflict-free 16-B reads)
-constexpr int kGtLen = 40;                           // gradient row length in LDS (80 B)
 
 int fail(int code, const std::string& msg) { return dxg::setError(code, msg); }
 
@@ -667,173 +664,314 @@ const void* rowsKernel(const ConvArgs& a)
 struct WgradArgs {
     const uint16_t* x;       // layer input
     const uint16_t* g;       // gradient of the layer's output (before its activation)
-    float* part;             // [grid][27][32 co][32 ci] partial sums
-    float* part_b;           // [grid][32]
+    float* part;             // [work-group][9 taps of its dz][32 co][32 ci] partial sums
+    float* part_b;           // [work-group][32], written where dz = 0
+    const uint16_t* zrow;    // voxel 0 of kZeroRow
     int nb, nz, ny, nx;
-    int units;               // nb*nz*(ny/4)*(nx/32)
-    int chunk;
+    int rows;                // rows of 64 voxels: nb*nz*ny*(nx/64)
 };
 
-__global__ __launch_bounds__(256) void wgrad_kernel(WgradArgs a)
+// A row of 64 voxels in the weight gradient's LDS: [phase][chunk][slot][8
+// channels] with voxel n of a phase in slot n + 1; slot 0 of phase 3 holds the
+// voxel before the row and slot 17 of phase 0 the one after.  A chunk takes 320
+// bytes: the two chunks and four voxels that a 16-lane group of a transposing
+// read covers then fall in distinct banks.
+constexpr int kWgChunk = 320, kWgPhase = 4 * kWgChunk, kWgRow = 4 * kWgPhase;
+constexpr int kWgWaves = 4;
+constexpr int kWgPart = 9 * 32 * 32;   // values of a work-group's partial sums
+static_assert(kWgPart * 4 <= kWgWaves * 2 * kWgRow, "the partial sums reuse the rows' LDS");
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+__device__ inline bf16x8 joinOperand(s16x4 lo, s16x4 hi)
 {
-    __shared__ __align__(16) uint16_t xT[18 * 32 * kXtLen];   // halo rows (dz, y) x channel x voxel: 64,512 B
-    __shared__ __align__(16) uint16_t gT[4 * 32 * kGtLen];    // 4 rows x channel x voxel: 10,240 B
-    __shared__ float bsh[32];
-    const int tid = threadIdx.x;
-    if (tid < 32)
-        bsh[tid] = 0.0f;
-    const int wave = tid >> 6, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
-    const int tap0 = wave * 7;
-    const int ntap = min(7, kTaps - tap0);
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
 
-    f32x4 acc[7][2][2];
-    for (int k = 0; k < 7; ++k)
-        for (int t = 0; t < 2; ++t)
-            for (int s = 0; s < 2; ++s)
-                acc[k][t][s] = f32x4 { 0, 0, 0, 0 };
-    float bsum = 0.0f;
+// Weight gradient.  A work-group takes the nine taps of one plane offset dz and
+// a range of rows per wavefront; a wavefront walks its rows along y with the
+// input rows of plane z + dz, and keeps 9 taps x 32 x 32 sums in registers (one
+// wavefront per SIMD, all 512 registers).  Step s applies input row y to the
+// gradient rows y + 1, y, y - 1 (taps dy = -1, 0, 1), so every row is read once
+// per dz.  K runs over voxels, the operands over channels, so rows pass through
+// LDS, private to the wavefront (no barriers), and come back by transposing
+// reads: 16 lanes get four voxels of 16 channels.  An operand is two phases
+// (32 voxels); the pairs (0,1) (2,3) (1,2) (0,3) of the gradient meet the input
+// pairs (0,1) (2,3) (-1,2) (1,4) so that the x offsets need no shifted reads
+// beyond phases -1 and 4.  While step s multiplies, the rows of step s + 1 go
+// through LDS and those of step s + 2 load.
+// CO, CI: channel halves with live values (the first layer's input and the last
+// layer's gradient have one; the other sums stay zero).
+// One layer on 4 x 64^3 voxels (58 GFLOP): 63 us, 920 TFLOP/s (73 us with the
+// compiler's own order of a step's instructions); a kernel that transposed rows
+// by two-byte LDS writes and read them back for each tap took 196 us, bound by
+// LDS.  What bounds it now: the matrix pipes and, as the variants with half of
+// the products still take 51 and 55 us, the three passes over x and g.
+template <int CO, int CI>
+__global__ __launch_bounds__(64 * kWgWaves) __attribute__((amdgpu_waves_per_eu(1, 1))) void wgrad_kernel(WgradArgs a)
+{
+    __shared__ __align__(16) unsigned char lds[kWgWaves * 2 * kWgRow];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+    // consecutive work-group ids alternate between the 8 XCDs: the three dz of
+    // a range of rows stay on one XCD, whose L2 then serves two of the three
+    const int i = blockIdx.x >> 3;
+    const int dz = i % 3 - 1;
+    const int wid = ((blockIdx.x & 7) * (gridDim.x / 24) + i / 3) * kWgWaves + wave, waves = gridDim.x / 3 * kWgWaves;
+    const int nxt = a.nx >> 6;
+    const ptrdiff_t row_stride = static_cast<ptrdiff_t>(a.nx) * kC;
+    const uint16_t* const zrow = a.zrow;
 
-    const int g = gridDim.x;
-    const int logical = (blockIdx.x & 7) * (g >> 3) + (blockIdx.x >> 3);
-    const int begin = logical * a.chunk;
-    const int end = min(begin + a.chunk, a.units);
-    const int nxc = a.nx >> 5, nyq = a.ny >> 2;
+    unsigned char* const xrow = lds + wave * 2 * kWgRow;
+    unsigned char* const grow = xrow + kWgRow;
+    const int wr_off = lq * kWgChunk + (lr + 1) * 16;
+    // where a lane writes its halo voxel: lanes 0 and 1 of a quarter the one
+    // before and after the row, the others each a slot of its own that nothing
+    // reads (18 and 19, 0 of phases 0-2, 17 of phases 1-3), so that the write
+    // needs no branch
+    const int halo_slot = lr < 2 ? 17 * lr : (lr < 10 ? 18 + (lr & 1) : (lr < 13 ? 0 : 17));
+    const int halo_phase = lr < 2 ? 3 - 3 * lr : (lr < 10 ? (lr - 2) >> 1 : (lr < 13 ? lr - 10 : lr - 12));
+    const int halo_off = halo_phase * kWgPhase + lq * kWgChunk + halo_slot * 16;
+    // transposing read: lane 4 k + c of a 16-lane group q addresses channels
+    // 4 c .. of voxel 4 q + k
+    const int tr_off = ((lr >> 1) & 1) * kWgChunk + (4 * lq + (lr >> 2) + 1) * 16 + (lr & 1) * 8;
+    auto readT = [&](const unsigned char* row, int off) {
+        typedef __attribute__((address_space(3))) s16x4* lds_ptr;
+        return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(row + tr_off + off));
+    };
 
-    for (int u = begin; u < end; ++u) {
-        int r = u / nxc;
-        const int x0 = (u - r * nxc) * 32;
-        const int y0 = (r % nyq) * 4;
-        r /= nyq;
-        const int z = r % a.nz;
-        const int n = r / a.nz;
-        __syncthreads();   // the previous tile is consumed
-        for (int i = tid; i < 4 * 32 * 4; i += 256) {
-            const int q = i & 3, vox = (i >> 2) & 31, rr = i >> 7;
-            const size_t row0 = (static_cast<size_t>(n * a.nz + z) * a.ny + y0 + rr) * a.nx;
-            const u32x4 d = load16(a.g + chunkAt(row0, x0 + vox, q));
-            uint16_t* dst = gT + (rr * 32 + 8 * q) * kGtLen + vox;
-            for (int e = 0; e < 4; ++e) {
-                dst[(2 * e) * kGtLen] = static_cast<uint16_t>(d[e] & 0xffffu);
-                dst[(2 * e + 1) * kGtLen] = static_cast<uint16_t>(d[e] >> 16);
+    f32x4 acc[9][CO][CI], accb[CO];
+#pragma unroll
+    for (int m = 0; m < CO; ++m) {
+        accb[m] = f32x4 { 0, 0, 0, 0 };
+#pragma unroll
+        for (int t = 0; t < 9; ++t)
+#pragma unroll
+            for (int k = 0; k < CI; ++k)
+                acc[t][m][k] = f32x4 { 0, 0, 0, 0 };
+    }
+    const bf16x8 ones = asOperand(u32x4 { 0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u });
+
+    const int r0 = static_cast<int>(static_cast<long long>(a.rows) * wid / waves);
+    const int r1 = static_cast<int>(static_cast<long long>(a.rows) * (wid + 1) / waves);
+    for (int r = r0; r < r1;) {
+        // the part of the range in one column (x tile of a plane)
+        const int col = r / a.ny, y0 = r - col * a.ny;
+        const int len = min(a.ny - y0, r1 - r);
+        r += len;
+        const int xt = col % nxt, plane = col / nxt, z = plane % a.nz;
+        if (static_cast<unsigned>(z + dz) >= static_cast<unsigned>(a.nz))
+            continue;
+        const uint16_t* const g0 = a.g + (static_cast<size_t>(plane) * a.ny + y0) * row_stride + static_cast<size_t>(xt) * kTile;
+        const uint16_t* const x0 = a.x + (static_cast<ptrdiff_t>(plane + dz) * a.ny + y0) * row_stride + static_cast<size_t>(xt) * kTile;
+        const bool left = xt > 0, right = xt + 1 < nxt;
+
+        u32x4 gw[4], xw[4], hw;          // rows on their way to LDS
+        bf16x8 gt[4][4][CO];             // gradient rows [ring][pair (0,1) (2,3) (1,2) (0,3)][half]
+        bf16x8 xt4[2][4][CI];            // input rows [ring][pair (0,1) (2,3) (-1,2) (1,4)][half]
+        // p where c, else the zero row; by masks, as a branch would end the
+        // region in which loads, LDS and matrix instructions interleave
+        auto rowOr0 = [&](bool c, const uint16_t* p) {
+            const uintptr_t m = uintptr_t(0) - static_cast<uintptr_t>(c);
+            return reinterpret_cast<const uint16_t*>((reinterpret_cast<uintptr_t>(p) & m) | (reinterpret_cast<uintptr_t>(zrow) & ~m));
+        };
+        // step s: input row y0 - 1 + s, gradient row y0 + s
+        auto load = [&](int s) {
+            const uint16_t* const gp = rowOr0(s < len, g0 + s * row_stride);
+            const int yx = y0 - 1 + s;
+            const bool in = static_cast<unsigned>(yx) < static_cast<unsigned>(a.ny);
+            const uint16_t* const xp = rowOr0(in, x0 + (s - 1) * row_stride);
+            const uint16_t* const lp = rowOr0(in && left, xp - kTile + 3 * kPhase + 15 * 8);
+            const uint16_t* const rp = rowOr0(in && right, xp + kTile);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                xw[j] = load16(xp + j * kPhase + lane * 8);
+                gw[j] = load16(gp + j * kPhase + lane * 8);
             }
-        }
-        for (int i = tid; i < 18 * 34 * 4; i += 256) {
-            const int q = i & 3, t = i >> 2;
-            const int row = t / 34, vox = t - row * 34;
-            const int zz = z + row / 6 - 1, yy = y0 + row % 6 - 1, xx = x0 + vox - 1;
-            u32x4 d = { 0, 0, 0, 0 };
-            if (static_cast<unsigned>(zz) < static_cast<unsigned>(a.nz) && static_cast<unsigned>(yy) < static_cast<unsigned>(a.ny)
-                && static_cast<unsigned>(xx) < static_cast<unsigned>(a.nx))
-                d = load16(a.x + chunkAt((static_cast<size_t>(n * a.nz + zz) * a.ny + yy) * a.nx, xx, q));
-            uint16_t* dst = xT + (row * 32 + 8 * q) * kXtLen + vox;
-            for (int e = 0; e < 4; ++e) {
-                dst[(2 * e) * kXtLen] = static_cast<uint16_t>(d[e] & 0xffffu);
-                dst[(2 * e + 1) * kXtLen] = static_cast<uint16_t>(d[e] >> 16);
+            hw = load16(((lr & 1) ? rp : lp) + lq * kChunk);
+        };
+        auto toLds = [&]() {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                *reinterpret_cast<u32x4*>(xrow + wr_off + j * kWgPhase) = xw[j];
+                *reinterpret_cast<u32x4*>(grow + wr_off + j * kWgPhase) = gw[j];
             }
+            *reinterpret_cast<u32x4*>(xrow + halo_off) = hw;
+            // one wavefront's LDS operations execute in program order: the
+            // fences only keep the compiler from moving reads over writes
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        };
+        auto fromLds = [&](bf16x8 (&xo)[4][CI], bf16x8 (&go)[4][CO]) {
+#pragma unroll
+            for (int k = 0; k < CI; ++k) {
+                const int h = k * 2 * kWgChunk;
+                const s16x4 m1 = readT(xrow, h + 3 * kWgPhase - 16), p0 = readT(xrow, h), p1 = readT(xrow, h + kWgPhase),
+                            p2 = readT(xrow, h + 2 * kWgPhase), p3 = readT(xrow, h + 3 * kWgPhase), p4 = readT(xrow, h + 16);
+                xo[0][k] = joinOperand(p0, p1);
+                xo[1][k] = joinOperand(p2, p3);
+                xo[2][k] = joinOperand(m1, p2);
+                xo[3][k] = joinOperand(p1, p4);
+            }
+#pragma unroll
+            for (int m = 0; m < CO; ++m) {
+                const int h = m * 2 * kWgChunk;
+                const s16x4 p0 = readT(grow, h), p1 = readT(grow, h + kWgPhase), p2 = readT(grow, h + 2 * kWgPhase),
+                            p3 = readT(grow, h + 3 * kWgPhase);
+                go[0][m] = joinOperand(p0, p1);
+                go[1][m] = joinOperand(p2, p3);
+                go[2][m] = joinOperand(p1, p2);
+                go[3][m] = joinOperand(p0, p3);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        };
+        const bf16x8 zero = asOperand(u32x4 { 0, 0, 0, 0 });
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int m = 0; m < CO; ++m)
+                gt[2][q][m] = gt[3][q][m] = zero;   // the two gradient rows before the range
+        load(0);
+        toLds();
+        load(1);
+        fromLds(xt4[0], gt[0]);
+        const int steps = len + 2;   // input rows y0 - 1 .. y0 + len
+        int s = 0;
+        auto step = [&](auto phase) {
+            constexpr int P = decltype(phase)::value;
+            toLds();             // the rows of step s + 1
+            load(s + 2);
+            fromLds(xt4[(P + 1) & 1], gt[(P + 1) & 3]);
+#pragma unroll
+            for (int dy = 0; dy < 3; ++dy) {   // gradient row y + 1 - dy
+                const bf16x8(&g)[4][CO] = gt[(P + 4 - dy) & 3];
+                const bf16x8(&x)[4][CI] = xt4[P & 1];
+                constexpr int gp[3][2] = { { 2, 3 }, { 0, 1 }, { 2, 3 } }, xp[3][2] = { { 0, 2 }, { 0, 1 }, { 1, 3 } };
+#pragma unroll
+                for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+                    for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                        for (int m = 0; m < CO; ++m)
+#pragma unroll
+                            for (int k = 0; k < CI; ++k)
+                                acc[3 * dy + dx][m][k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g[gp[dx][k2]][m], x[xp[dx][k2]][k],
+                                                                                             acc[3 * dy + dx][m][k], 0, 0, 0);
+            }
+            // the order in which the step's instructions issue: an LDS write,
+            // a load or a read between every one or two matrix instructions
+            // (the compiler groups them and the matrix pipe waits)
+#pragma unroll
+            for (int k = 0; k < 9; ++k) {
+                __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);   // LDS write
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // matrix
+            }
+#pragma unroll
+            for (int k = 0; k < 9; ++k) {
+                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);   // load
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            }
+#pragma unroll
+            for (int k = 0; k < 20; ++k) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
+                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            }
+            if (dz == 0) {   // bias gradient: the sum over the gradient row of step s
+#pragma unroll
+                for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+                    for (int m = 0; m < CO; ++m)
+                        accb[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gt[P & 3][k2][m], ones, accb[m], 0, 0, 0);
+            }
+            ++s;
+        };
+        for (;;) {
+            step(std::integral_constant<int, 0> {});
+            if (s == steps)
+                break;
+            step(std::integral_constant<int, 1> {});
+            if (s == steps)
+                break;
+            step(std::integral_constant<int, 2> {});
+            if (s == steps)
+                break;
+            step(std::integral_constant<int, 3> {});
+            if (s == steps)
+                break;
         }
+    }
+
+    // the work-group's sums, its wavefronts added in order
+    float* const sum = reinterpret_cast<float*>(lds);
+    float* const part = a.part + static_cast<size_t>(blockIdx.x) * kWgPart;
+    for (int w = 0; w < kWgWaves; ++w) {
         __syncthreads();
-        if (tid < 128) {
-            const uint16_t* s = gT + ((tid >> 5) * 32 + (tid & 31)) * kGtLen;
-            for (int v = 0; v < 32; ++v)
-                bsum += fromBf16(s[v]);
+        if (wave == w) {
+#pragma unroll
+            for (int t = 0; t < 9; ++t)
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+#pragma unroll
+                    for (int k = 0; k < 2; ++k)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            float* const d = sum + (t * 32 + 16 * m + 4 * lq + e) * 32 + 16 * k + lr;
+                            const float v = m < CO && k < CI ? acc[t][m < CO ? m : 0][k < CI ? k : 0][e] : 0.0f;
+                            *d = w == 0 ? v : *d + v;
+                        }
         }
-        for (int rr = 0; rr < 4; ++rr) {
-            bf16x8 ga[2];
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-                ga[t] = asOperand(load16(gT + (rr * 32 + 16 * t + lr) * kGtLen + 8 * lq));
-#pragma unroll
-            for (int k = 0; k < 7; ++k) {
-                if (k >= ntap)
-                    break;
-                const int tap = tap0 + k;
-                const int dzi = tap / 9, dyi = (tap / 3) % 3, dxi = tap % 3;
-                const int row = dzi * 6 + rr + dyi;
-#pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    const uint16_t* p = xT + (row * 32 + 16 * s + lr) * kXtLen + 8 * lq;
-                    const u32x4 lo = load16(p), hi = load16(p + 8);
-                    u32x4 b;
-                    if (dxi == 0) {
-                        b = lo;
-                    } else if (dxi == 1) {
-                        b = u32x4 { __builtin_amdgcn_alignbyte(lo[1], lo[0], 2), __builtin_amdgcn_alignbyte(lo[2], lo[1], 2),
-                                    __builtin_amdgcn_alignbyte(lo[3], lo[2], 2), __builtin_amdgcn_alignbyte(hi[0], lo[3], 2) };
-                    } else {
-                        b = u32x4 { lo[1], lo[2], lo[3], hi[0] };
-                    }
-                    const bf16x8 bop = asOperand(b);
-#pragma unroll
-                    for (int t = 0; t < 2; ++t)
-                        acc[k][t][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga[t], bop, acc[k][t][s], 0, 0, 0);
-                }
-            }
-        }
-    }
-
-    float* part = a.part + static_cast<size_t>(blockIdx.x) * kLayerW;
-#pragma unroll
-    for (int k = 0; k < 7; ++k) {
-        if (k >= ntap)
-            break;
-        const int tap = tap0 + k;
-        for (int t = 0; t < 2; ++t)
-            for (int s = 0; s < 2; ++s)
-                for (int i = 0; i < 4; ++i)
-                    part[(tap * 32 + 16 * t + 4 * lq + i) * 32 + 16 * s + lr] = acc[k][t][s][i];
     }
     __syncthreads();
-    if (tid < 128)
-        atomicAdd(&bsh[tid & 31], bsum);
+    for (int k = tid; k < kWgPart; k += 64 * kWgWaves)
+        part[k] = sum[k];
+    if (dz != 0)
+        return;
+    for (int w = 0; w < kWgWaves; ++w) {
+        __syncthreads();
+        if (wave == w && lr == 0) {
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float* const d = sum + 16 * m + 4 * lq + e;
+                    const float v = m < CO ? accb[m < CO ? m : 0][e] : 0.0f;
+                    *d = w == 0 ? v : *d + v;
+                }
+        }
+    }
     __syncthreads();
     if (tid < 32)
-        a.part_b[static_cast<size_t>(blockIdx.x) * 32 + tid] = bsh[tid];
+        a.part_b[static_cast<size_t>(blockIdx.x) * 32 + tid] = sum[tid];
 }
 
-// Sum the per-work-group partials into one layer's gradient, in two fixed-
-// order stages: slice y of the partials into sums[y], then the slices into the
-// parameter layout ([co][tap][ci] weights, then 32 biases).
-constexpr int kReduceSlices = 8;
+// Adds the work-groups' partials of one layer in a fixed order (four slices of
+// work-groups, then the slices) into the parameter layout ([co][tap][ci]
+// weights, then 32 biases).  One work-group per 64 values.
+constexpr int kReduceBlocks = kLayerW / 64 + 1;   // the last one takes the biases
 
-__global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* part, const float* part_b, int parts, float* sums)
+__global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* part, const float* part_b, int groups, float* grad)
 {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    const int per = (parts + kReduceSlices - 1) / kReduceSlices;
-    const int p0 = blockIdx.y * per, p1 = min(parts, p0 + per);
-    if (i < kLayerW) {
-        float s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-        int p = p0;
-        for (; p + 4 <= p1; p += 4) {
-            s0 += part[static_cast<size_t>(p) * kLayerW + i];
-            s1 += part[static_cast<size_t>(p + 1) * kLayerW + i];
-            s2 += part[static_cast<size_t>(p + 2) * kLayerW + i];
-            s3 += part[static_cast<size_t>(p + 3) * kLayerW + i];
-        }
-        for (; p < p1; ++p)
-            s0 += part[static_cast<size_t>(p) * kLayerW + i];
-        sums[blockIdx.y * kLayerP + i] = (s0 + s1) + (s2 + s3);
-    } else if (i < kLayerP) {
-        const int co = i - kLayerW;
-        float s = 0;
-        for (int p = p0; p < p1; ++p)
-            s += part_b[p * 32 + co];
-        sums[blockIdx.y * kLayerP + i] = s;
+    __shared__ float slice[4][64];
+    const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const bool bias = blockIdx.x == kLayerW / 64;
+    const int v = blockIdx.x * 64 + lane;                    // [tap][co][ci]
+    const int dz = bias ? 1 : v / kWgPart;                   // plane offset 0..2
+    const float* const src = bias ? part_b + (lane & 31) : part + (v - dz * kWgPart);
+    const int stride = bias ? 32 : kWgPart;
+    // work-group b = 8 i + xcd holds dz = i % 3
+    const int n = groups / 3, per = (n + 3) / 4, k1 = min(n, (q + 1) * per);
+    float s = 0.0f;
+    for (int k = q * per; k < k1; ++k) {
+        const int b = 8 * (3 * (k >> 3) + dz) + (k & 7);
+        s += src[static_cast<size_t>(b) * stride];
     }
-}
-
-__global__ __launch_bounds__(256) void wgrad_finish_kernel(const float* sums, float* grad)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= kLayerP)
+    slice[q][lane] = s;
+    __syncthreads();
+    if (q != 0)
         return;
-    float s = 0;
-    for (int k = 0; k < kReduceSlices; ++k)
-        s += sums[k * kLayerP + i];
-    if (i < kLayerW) {
-        const int tap = i >> 10, co = (i >> 5) & 31, ci = i & 31;
+    s = (slice[0][lane] + slice[1][lane]) + (slice[2][lane] + slice[3][lane]);
+    if (!bias) {
+        const int tap = v >> 10, co = (v >> 5) & 31, ci = v & 31;
         grad[(co * kTaps + tap) * kC + ci] = s;
-    } else {
-        grad[i] = s;
+    } else if (lane < 32) {
+        grad[kLayerW + lane] = s;
     }
 }
 
@@ -1134,13 +1272,18 @@ hipError_t launchConv(ConvArgs a, const Dims& d, hipStream_t s)
     return hipGetLastError();
 }
 
+// Work-groups of the weight gradient: one per CU (a wavefront takes a SIMD's
+// registers), a multiple of 24 (three dz on each of 8 XCDs); fewer where a
+// wavefront would get less than eight rows (it reads two more than it has).
 int wgradGrid(const Dims& d)
 {
-    const int units = d.nb * d.nz * (d.ny / 4) * (d.nx / 32);
-    return roundUp8(std::min(units, 2 * computeUnits()));
+    const long long rows = static_cast<long long>(d.nb) * d.nz * d.ny * (d.nx / 64);
+    const long long want = (rows + 8 * kWgWaves * 8 - 1) / (8 * kWgWaves * 8);   // groups of 24 with eight rows a wavefront
+    return 24 * static_cast<int>(std::min<long long>(want, std::max(1, computeUnits() / 24)));
 }
 
-hipError_t launchWgrad(const uint16_t* x, const uint16_t* g, float* part, float* part_b, float* sums, float* grad, const Dims& d,
+// live: channels of x and g that can hold values other than zero.
+hipError_t launchWgrad(const uint16_t* x, int x_live, const uint16_t* g, int g_live, float* part, float* part_b, float* grad, const Dims& d,
                        hipStream_t s)
 {
     WgradArgs a {};
@@ -1148,16 +1291,22 @@ hipError_t launchWgrad(const uint16_t* x, const uint16_t* g, float* part, float*
     a.g = g;
     a.part = part;
     a.part_b = part_b;
+    a.zrow = zeroRow();
+    if (!a.zrow)
+        return hipErrorInvalidSymbol;
     a.nb = d.nb;
     a.nz = d.nz;
     a.ny = d.ny;
     a.nx = d.nx;
-    a.units = d.nb * d.nz * (d.ny / 4) * (d.nx / 32);
+    a.rows = d.nb * d.nz * d.ny * (d.nx / 64);
     const int grid = wgradGrid(d);
-    a.chunk = (a.units + grid - 1) / grid;
-    hipLaunchKernelGGL(wgrad_kernel, dim3(grid), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((kLayerP + 255) / 256, kReduceSlices), dim3(256), 0, s, part, part_b, grid, sums);
-    hipLaunchKernelGGL(wgrad_finish_kernel, dim3((kLayerP + 255) / 256), dim3(256), 0, s, sums, grad);
+    if (g_live <= 16)
+        hipLaunchKernelGGL((wgrad_kernel<1, 2>), dim3(grid), dim3(64 * kWgWaves), 0, s, a);
+    else if (x_live <= 16)
+        hipLaunchKernelGGL((wgrad_kernel<2, 1>), dim3(grid), dim3(64 * kWgWaves), 0, s, a);
+    else
+        hipLaunchKernelGGL((wgrad_kernel<2, 2>), dim3(grid), dim3(64 * kWgWaves), 0, s, a);
+    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(kReduceBlocks), dim3(256), 0, s, part, part_b, grid, grad);
     return hipGetLastError();
 }
 
@@ -1426,7 +1575,7 @@ struct dxg_denoiser {
     DBuf<float> params, adam_m, adam_v, grads;
     DBuf<uint16_t> wf, wd;
     DBuf<uint16_t> xin, xin4, acts, gbuf;
-    DBuf<float> feat0, y32, target, mask, features, lpart, part, part_b, sums, wemb;
+    DBuf<float> feat0, y32, target, mask, features, lpart, part, part_b, wemb;
     DBuf<double> wacc, wdose;
     DBuf<int> tiles;                    // kLayers lists of up to tiles_stride entries, layer l's at l * tiles_stride
     size_t tiles_stride = 0;
@@ -1667,11 +1816,10 @@ struct dxg_denoiser {
         uint16_t* gs = gbuf.p + ts;
         uint16_t* gh = gbuf.p + 2 * ts;
         const int grid = wgradGrid(d);
-        HIP_TRY(part.reserve(static_cast<size_t>(grid) * kLayerW));
+        HIP_TRY(part.reserve(static_cast<size_t>(grid) * kWgPart));
         HIP_TRY(part_b.reserve(static_cast<size_t>(grid) * 32));
-        HIP_TRY(sums.reserve(static_cast<size_t>(kReduceSlices) * kLayerP));
 
-        HIP_TRY(launchWgrad(aT(kBlocks), gout, part.p, part_b.p, sums.p, layerGrad(kLayers - 1), d, stream));
+        HIP_TRY(launchWgrad(aT(kBlocks), kC, gout, 1, part.p, part_b.p, layerGrad(kLayers - 1), d, stream));
         ConvArgs c {};
         c.x = gout;
         c.w = layerWd(kLayers - 1);
@@ -1679,14 +1827,14 @@ struct dxg_denoiser {
         c.y = gs;
         HIP_TRY(launchConv(c, d, stream));
         for (int b = kBlocks - 1; b >= 0; --b) {
-            HIP_TRY(launchWgrad(hT(b), gs, part.p, part_b.p, sums.p, layerGrad(2 * b + 2), d, stream));
+            HIP_TRY(launchWgrad(hT(b), kC, gs, kC, part.p, part_b.p, layerGrad(2 * b + 2), d, stream));
             c = ConvArgs {};
             c.x = gs;
             c.w = layerWd(2 * b + 2);
             c.gate = hT(b);
             c.y = gh;
             HIP_TRY(launchConv(c, d, stream));
-            HIP_TRY(launchWgrad(aT(b), gh, part.p, part_b.p, sums.p, layerGrad(2 * b + 1), d, stream));
+            HIP_TRY(launchWgrad(aT(b), kC, gh, kC, part.p, part_b.p, layerGrad(2 * b + 1), d, stream));
             c = ConvArgs {};
             c.x = gh;
             c.w = layerWd(2 * b + 1);
@@ -1695,7 +1843,7 @@ struct dxg_denoiser {
             c.y = gs;
             HIP_TRY(launchConv(c, d, stream));
         }
-        HIP_TRY(launchWgrad(xin.p, gs, part.p, part_b.p, sums.p, layerGrad(0), d, stream));
+        HIP_TRY(launchWgrad(xin.p, DXG_DENOISE_FEATURES, gs, kC, part.p, part_b.p, layerGrad(0), d, stream));
         return DXG_OK;
     }
 };
@@ -2084,12 +2232,10 @@ int dxg_conv3d_probe(int mode, const float* x, const float* w, const float* bias
         HIP_TRY(dy.reserve(ts));
         HIP_TRY(hipMemcpy(dy.p, gh.data(), ts * 2, hipMemcpyHostToDevice));
         const int grid = wgradGrid(dm);
-        HIP_TRY(part.reserve(static_cast<size_t>(grid) * kLayerW));
+        HIP_TRY(part.reserve(static_cast<size_t>(grid) * kWgPart));
         HIP_TRY(part_b.reserve(static_cast<size_t>(grid) * 32));
         HIP_TRY(dout.reserve(kLayerP));
-        DBuf<float> sums;
-        HIP_TRY(sums.reserve(static_cast<size_t>(kReduceSlices) * kLayerP));
-        HIP_TRY(launchWgrad(dx.p, dy.p, part.p, part_b.p, sums.p, dout.p, dm, nullptr));
+        HIP_TRY(launchWgrad(dx.p, kC, dy.p, kC, part.p, part_b.p, dout.p, dm, nullptr));
         HIP_TRY(hipMemcpy(out, dout.p, kLayerP * sizeof(float), hipMemcpyDeviceToHost));
         return DXG_OK;
     }

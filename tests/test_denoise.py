@@ -221,6 +221,30 @@ def test_conv_weight_grad_matches_torch(n, dims):
     np.testing.assert_allclose(out, want, rtol=0, atol=5e-5 * np.abs(want).max())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,dims", [(1, (2, 4, 64)), (2, (3, 12, 192)), (1, (1, 36, 128)), (3, (9, 28, 64)), (1, (33, 68, 128))])
+def test_conv_weight_grad_rows_and_edges(n, dims):
+    """The weight gradient where its row ranges begin and end: fewer rows than
+    wavefronts, x tiles with neighbours on no, one and both sides, one plane
+    (two of three plane offsets outside), ranges that cross columns, planes and
+    volumes, and more rows than one range a wavefront."""
+    x, w, _ = _conv_inputs(17, n, dims)
+    rng = np.random.default_rng(18)
+    g = rng.normal(0.0, 1.0, x.shape).astype(np.float32)
+    out = _probe(2, x, w.reshape(-1), g, n, dims)
+    xd, gd = torch.from_numpy(_bf16(x)).double(), torch.from_numpy(_bf16(g)).double()
+    xp = torch.nn.functional.pad(xd, (0, 0, 1, 1, 1, 1, 1, 1))
+    d, h, wd = dims
+    want = np.stack([(gd.reshape(-1, 32).t() @ xp[:, a:a + d, b:b + h, c:c + wd].reshape(-1, 32)).numpy()
+                     for a in range(3) for b in range(3) for c in range(3)], axis=1)
+    # FP32 sums of up to 3e5 products of unit variance in 320 ranges: each adds
+    # about 1e3 terms, so rounding stays near 1e3 * 2^-24 = 6e-5 of a range's
+    # sum and, the ranges' errors being independent, below 1e-5 of the total
+    np.testing.assert_allclose(out[:27648].reshape(32, 27, 32), want, rtol=0, atol=1e-5 * np.abs(want).max())
+    db = gd.reshape(-1, 32).sum(0).numpy()
+    np.testing.assert_allclose(out[27648:27680], db, rtol=0, atol=1e-5 * max(np.abs(db).max(), np.sqrt(gd.numel() / 32)))
+
+
 def _net_case(seed, batch, dims):
     rng = np.random.default_rng(seed)
     f = np.empty((batch,) + dims + (4,), dtype=np.float32)

@@ -34,7 +34,7 @@ HIP_FLAGS = [
     "-Wall", "-Wno-unused-command-line-argument",
     f"-I{ROOT / 'include'}", f"-I{CSRC}",
 ]
-SOURCES = ["physics.cpp", "world.cpp", "beams.cpp", "calibration.cpp", "batch.cpp", "transport.hip", "denoise.hip", "pipelines.hip",
+SOURCES = ["physics.cpp", "world.cpp", "beams.cpp", "calibration.cpp", "batch.cpp", "hostio.cpp", "transport.hip", "denoise.hip", "pipelines.hip",
            "h5io.cpp"]
 # h5io.cpp compiles against the HDF5 headers only; the library itself is
 # opened with dlopen when a project file is first touched.

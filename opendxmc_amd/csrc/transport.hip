@@ -1318,6 +1318,26 @@ __global__ void tally_fold_kernel(double* __restrict__ t, unsigned long long str
     }
 }
 
+// Tally records to separate arrays, written over PCIe into pinned host memory:
+// bound by the link, 55 GB/s of 24 bytes a voxel (a copy engine moves whole
+// 32-byte records at 56 GB/s, and the host had to take them apart).
+__global__ __launch_bounds__(256) void scores_kernel(const double* __restrict__ tally, uint64_t n, double* __restrict__ sum_e,
+                                                     double* __restrict__ sum_e2, uint64_t* __restrict__ events)
+{
+    const uint64_t v = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (v >= n)
+        return;
+    static_assert(kTallyRecord == 4, "two 16-byte loads a record");
+    const double2* rec = reinterpret_cast<const double2*>(tally) + 2 * v;
+    const double2 a = rec[0], b = rec[1];
+    if (sum_e)
+        sum_e[v] = a.x;
+    if (sum_e2)
+        sum_e2[v] = a.y;
+    if (events)   // an FP64 integer (exact below 2^53)
+        events[v] = static_cast<uint64_t>(b.x);
+}
+
 __global__ void reset_kernel(unsigned long long* pool, DevCounters* c)
 {
     if (threadIdx.x == 0) {
@@ -1435,6 +1455,13 @@ void launchTallyFold(double* tally, unsigned long long stride, int replicas, hip
     const unsigned long long want = (stride + 255) / 256;
     const unsigned blocks = static_cast<unsigned>(std::min<unsigned long long>(want, 8192));
     hipLaunchKernelGGL(tally_fold_kernel, dim3(blocks), dim3(256), 0, s, tally, stride, replicas);
+}
+
+void launchScores(const double* tally, uint64_t n, double* sum_e, double* sum_e2, uint64_t* events, hipStream_t s)
+{
+    if (n == 0)
+        return;
+    hipLaunchKernelGGL(scores_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s, tally, n, sum_e, sum_e2, events);
 }
 
 void launchReset(unsigned long long* pool, DevCounters* counters, hipStream_t s)

@@ -99,7 +99,7 @@ class Denoiser:
         f = np.ascontiguousarray(features, dtype=np.float32)
         if f.ndim != 4 or f.shape[-1] != FEATURES:
             raise ValueError("features must be (D, H, W, 4)")
-        out = np.zeros(f.shape[:3], dtype=np.float32)
+        out = np.empty(f.shape[:3], dtype=np.float32)
         dims = np.array(f.shape[:3], dtype=np.uint64)
         N.check(N.lib().dxg_denoiser_infer(self._h, _pf(f), dims.ctypes.data_as(C.POINTER(N.u64)), _pf(out)))
         return out
@@ -113,14 +113,14 @@ class Denoiser:
         (nz, ny, nx padded to 64, 4)."""
         nx, ny, nz = grid.dims
         nxp = (nx + 63) // 64 * 64
-        f = np.zeros((nz, ny, nxp, FEATURES), dtype=np.float32)
+        f = np.empty((nz, ny, nxp, FEATURES), dtype=np.float32)
         N.check(N.lib().dxg_denoiser_world_features(self._h, grid._h, _pf(f), f.size))
         return f
 
     def apply(self, grid, copy_out: bool = True) -> np.ndarray | None:
         """Denoise a grid's current dose on the device; returns the dose (mGy,
         flat grid order) unless copy_out is False (device timing only)."""
-        out = np.zeros(grid.size(), dtype=np.float64) if copy_out else None
+        out = np.empty(grid.size(), dtype=np.float64) if copy_out else None
         p = out.ctypes.data_as(C.POINTER(C.c_double)) if copy_out else None
         N.check(N.lib().dxg_denoiser_apply(self._h, grid._h, p))
         return out

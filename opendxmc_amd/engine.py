@@ -147,14 +147,14 @@ class AAVoxelGrid:
     def energyScored(self):
         """(sum w dE keV, sum (w dE)^2 keV^2, events) per voxel."""
         n = self.size()
-        e, e2, ev = np.zeros(n), np.zeros(n), np.zeros(n, dtype=np.uint64)
+        e, e2, ev = np.empty(n), np.empty(n), np.empty(n, dtype=np.uint64)
         N.check(N.lib().dxg_read_energy_scores(self._h, N.ptr(e, C.c_double), N.ptr(e2, C.c_double), N.ptr(ev, N.u64)))
         return e, e2, ev
 
     def doseScored(self):
         """(dose mGy, variance mGy^2, numberOfEvents) per voxel (DoseScore)."""
         n = self.size()
-        d, v, ev = np.zeros(n), np.zeros(n), np.zeros(n, dtype=np.uint64)
+        d, v, ev = np.empty(n), np.empty(n), np.empty(n, dtype=np.uint64)
         N.check(N.lib().dxg_read_dose_scores(self._h, N.ptr(d, C.c_double), N.ptr(v, C.c_double), N.ptr(ev, N.u64)))
         return d, v, ev
 

@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <numeric>
 #include <string>
 #include <vector>
@@ -218,6 +219,11 @@ int dxg_batch_run(dxg_batch* b, double* kernel_ms)
     int cus = 0;
     HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device));
     const int blocks = cus * dxg::transportBatchBlocksPerCU(lut, level, cells, lds);
+    if (!std::getenv("DXG_BATCH")) {   // each instance's share of the work-groups is in proportion to its histories
+        const double all = std::accumulate(work.begin(), work.end(), 0.0);
+        for (auto& p : ps)
+            p.batch = dxg::claimSize(static_cast<unsigned long long>(all), blocks);
+    }
     // initial block -> instance assignment proportional to each instance's histories
     std::vector<int> start(static_cast<size_t>(blocks));
     const double tot = std::accumulate(work.begin(), work.end(), 0.0);
@@ -282,15 +288,15 @@ int dxg_batch_run(dxg_batch* b, double* kernel_ms)
     HIP_TRY(hipEventRecord(b->ev0, b->stream));
     HIP_TRY(hipGraphLaunch(b->exec, b->stream));
     HIP_TRY(hipEventRecord(b->ev1, b->stream));
-    std::vector<dxg::DevCounters> cs(static_cast<size_t>(n));
+    std::vector<dxg::DevCounters> cs(static_cast<size_t>(n) * dxg::kCounterCopies);
     for (int i = 0; i < n; ++i)
-        HIP_TRY(hipMemcpyAsync(&cs[static_cast<size_t>(i)], ps[static_cast<size_t>(i)].counters, sizeof(dxg::DevCounters),
-                               hipMemcpyDeviceToHost, b->stream));
+        HIP_TRY(hipMemcpyAsync(&cs[static_cast<size_t>(i) * dxg::kCounterCopies], ps[static_cast<size_t>(i)].counters,
+                               sizeof(dxg::DevCounters) * dxg::kCounterCopies, hipMemcpyDeviceToHost, b->stream));
     HIP_TRY(hipStreamSynchronize(b->stream));
     float ms = 0.0f;
     HIP_TRY(hipEventElapsedTime(&ms, b->ev0, b->ev1));
     for (int i = 0; i < n; ++i) {
-        const dxg::DevCounters& c = cs[static_cast<size_t>(i)];
+        const dxg::DevCounters c = dxg::sumCounters(&cs[static_cast<size_t>(i) * dxg::kCounterCopies]);
         dxg_counters acc {};
         acc.histories = c.histories;
         acc.steps = c.steps;

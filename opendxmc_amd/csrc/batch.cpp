@@ -78,6 +78,7 @@ struct dxg_batch {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     dxg::DevParams* d_params = nullptr;
+    dxg::DevCounters* d_counters = nullptr;   // of every instance
     int* d_start = nullptr;
     size_t cap = 0, start_cap = 0;
     hipGraph_t graph = nullptr;
@@ -103,6 +104,8 @@ struct dxg_batch {
         dropGraph();
         if (d_params)
             (void)hipFree(d_params);
+        if (d_counters)
+            (void)hipFree(d_counters);
         if (d_start)
             (void)hipFree(d_start);
         if (ev0)
@@ -243,7 +246,12 @@ int dxg_batch_run(dxg_batch* b, double* kernel_ms)
         if (b->d_params)
             (void)hipFree(b->d_params);
         b->d_params = nullptr;
+        if (b->d_counters)
+            (void)hipFree(b->d_counters);
+        b->d_counters = nullptr;
+        b->cap = 0;
         HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->d_params), sizeof(dxg::DevParams) * static_cast<size_t>(n)));
+        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&b->d_counters), sizeof(dxg::DevCounters) * dxg::kCounterCopies * static_cast<size_t>(n)));
         b->cap = static_cast<size_t>(n);
         b->dropGraph();
     }
@@ -288,10 +296,10 @@ int dxg_batch_run(dxg_batch* b, double* kernel_ms)
     HIP_TRY(hipEventRecord(b->ev0, b->stream));
     HIP_TRY(hipGraphLaunch(b->exec, b->stream));
     HIP_TRY(hipEventRecord(b->ev1, b->stream));
+    dxg::launchBatchFinish(b->d_params, n, b->d_counters, b->stream);
+    HIP_TRY(hipGetLastError());
     std::vector<dxg::DevCounters> cs(static_cast<size_t>(n) * dxg::kCounterCopies);
-    for (int i = 0; i < n; ++i)
-        HIP_TRY(hipMemcpyAsync(&cs[static_cast<size_t>(i) * dxg::kCounterCopies], ps[static_cast<size_t>(i)].counters,
-                               sizeof(dxg::DevCounters) * dxg::kCounterCopies, hipMemcpyDeviceToHost, b->stream));
+    HIP_TRY(hipMemcpyAsync(cs.data(), b->d_counters, cs.size() * sizeof(dxg::DevCounters), hipMemcpyDeviceToHost, b->stream));
     HIP_TRY(hipStreamSynchronize(b->stream));
     float ms = 0.0f;
     HIP_TRY(hipEventElapsedTime(&ms, b->ev0, b->ev1));
@@ -315,8 +323,6 @@ int dxg_batch_run(dxg_batch* b, double* kernel_ms)
         acc.kernel_ms = ms;          // the shared launch
         acc.kernel_launches = 1;
         dxg::addHistories(b->inst[static_cast<size_t>(i)].world, b->inst[static_cast<size_t>(i)].histories, acc);
-        if (int rc = dxg::foldTally(b->inst[static_cast<size_t>(i)].world); rc != DXG_OK)
-            return rc;
     }
     if (kernel_ms)
         *kernel_ms = ms;

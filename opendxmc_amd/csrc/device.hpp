@@ -236,6 +236,9 @@ void launchTraverse(const DevParams& p, uint64_t n_rays, const float* pos, const
 void launchReset(unsigned long long* pool, DevCounters* counters, hipStream_t s);
 // Adds tally copies 1..replicas-1 into copy 0 (in that order) and zeroes them.
 void launchTallyFold(double* tally, unsigned long long stride, int replicas, hipStream_t s);
+// The same for every instance of a batch run, and their counters (kCounterCopies
+// each) to `out`, in one launch; params and out are device arrays.
+void launchBatchFinish(const DevParams* params, int n_inst, DevCounters* out, hipStream_t s);
 // The scores of voxels [0, n) of `tally` (records of kTallyRecord doubles) as
 // arrays: sum w dE and sum (w dE)^2 as doubles, the events as integers; each to
 // its array unless null.  The arrays may be device-accessible host memory.
@@ -279,9 +282,6 @@ int staticScratch(int device, void** out);
 // beam, uploads its tables to the world and fills p (all but the history
 // range); total receives the beam's history count.
 int prepareRun(dxg_world* w, const dxg_beam* beam, uint64_t seed, DevParams& p, uint64_t& total);
-// Folds the world's tally copies into one after a run (no-op with one copy);
-// enqueued on the world's stream.
-int foldTally(dxg_world* w);
 // After a run outside dxg_transport_run: account n histories and set the counters.
 void addHistories(dxg_world* w, uint64_t n, const dxg_counters& c);
 int worldDevice(const dxg_world* w);

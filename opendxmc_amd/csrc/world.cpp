@@ -498,10 +498,13 @@ int dxg_world_build(dxg_world* w)
     // are applied one after another where the memory holds it, so a narrow
     // beam on a small grid (a pencil beam's axis voxels take most first
     // interactions) waits on a few records; work-groups spread over the copies
-    // and a fold after each run sums them.  Up to 16 copies within 128 MiB.
+    // and a fold after each run sums them.  Up to 8 copies within 128 MiB: a
+    // call with a pencil beam into 64^3 water took, with 1 / 2 / 4 / 8 / 16
+    // copies, 0.40 / 0.25 / 0.228 / 0.225 / 0.235 ms at 1e6 histories and 25.9 /
+    // 9.1 / 6.25 / 5.99 / 6.41 ms at 1e8 (16 copies fall out of the caches).
     {
         const size_t bytes = w->tallyDoubles() * sizeof(double);
-        w->replicas = static_cast<int>(std::clamp<size_t>((size_t(128) << 20) / std::max<size_t>(bytes, 1), 1, 16));
+        w->replicas = static_cast<int>(std::clamp<size_t>((size_t(128) << 20) / std::max<size_t>(bytes, 1), 1, 8));
         if (const char* env = std::getenv("DXG_TALLY_REPLICAS"))
             w->replicas = std::clamp(std::atoi(env), 1, 64);
     }
@@ -805,15 +808,6 @@ void addHistories(dxg_world* w, uint64_t n, const dxg_counters& c)
 }
 
 int worldDevice(const dxg_world* w) { return w->device; }
-
-int foldTally(dxg_world* w)
-{
-    HIP_TRY(hipSetDevice(w->device));
-    dxg::launchTallyFold(w->d_tally.ptr, w->tallyDoubles(), w->replicas, w->stream);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(w->stream));
-    return DXG_OK;
-}
 
 // Launch settings chosen by the run's own timing, kept per world build and
 // beam layout: dead lanes that start a refill, parked lanes that start an

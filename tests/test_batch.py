@@ -65,3 +65,37 @@ def test_batch_equals_one_run_per_instance():
             np.testing.assert_allclose(e2, e1, rtol=1e-10, atol=1e-12 * e1.max())
             np.testing.assert_allclose(e22, e21, rtol=1e-10, atol=1e-12 * e21.max())
             assert c2["deposited_energy"] == pytest.approx(c1["deposited_energy"], rel=1e-12)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("copies", [2, 4, 5, 8, 11])
+def test_tally_copies_fold_to_the_single_copy(copies, monkeypatch):
+    """Worlds with several tally copies (whole and partial groups of four),
+    folded by a plain call and by a batch run, against worlds with one; twice,
+    so that copies left unzeroed would count again.  A voxel's sums hold the
+    same terms in another order: within 2 * events * 2^-53."""
+    inst = bw.instances(3, seed=11, shape_scale=0.2, hist_range=(5e4, 2e5))
+    monkeypatch.setenv("DXG_TALLY_REPLICAS", "1")
+    plain = [bw.make_world(ph) for ph, _, _ in inst]
+    monkeypatch.setenv("DXG_TALLY_REPLICAS", str(copies))
+    single = [bw.make_world(ph) for ph, _, _ in inst]
+    batched = [bw.make_world(ph) for ph, _, _ in inst]
+    batch = dx.TransportBatch()
+    for (ph, beam, s), (world, _) in zip(inst, batched):
+        batch.add(world, beam, s)
+    for _ in range(2):
+        tr = dx.Transport()
+        for worlds in (plain, single):
+            for (ph, beam, s), (world, _) in zip(inst, worlds):
+                tr.seed = s
+                tr(world, beam, None, True)
+        batch.run()
+        for (_, g0), (_, g1), (_, g2) in zip(plain, single, batched):
+            e, e2, ev = g0.energyScored()
+            assert ev.sum() > 0
+            for g in (g1, g2):
+                f, f2, fv = g.energyScored()
+                np.testing.assert_array_equal(fv, ev)
+                assert np.all(np.abs(f - e) <= 2 * ev * 2.0**-53 * e)
+                assert np.all(np.abs(f2 - e2) <= 2 * ev * 2.0**-53 * e2)
+                assert all(g.counters()[name] == g0.counters()[name] for name in COUNTS)

@@ -102,6 +102,11 @@ __device__ inline u32x4 load16(const uint16_t* p) { return *reinterpret_cast<con
 // 16 voxels of a phase is contiguous: [phase j][chunk q][voxel n][8 channels].
 // A matrix operand of one phase (16 voxels x 32 channels, lane 16 q + n holding
 // chunk q of voxel n) is then one contiguous kilobyte read in lane order.
+// With a voxel's 32 channels contiguous instead, each 16-lane pass of a load
+// fell in 16 cache lines and the texture address units were 95 % busy: 18
+// layers of 128x256x256 voxels 11.1 ms, so 8.4 (8.2 with the weights straight to
+// LDS: 985 TFLOP/s a full layer, where a library product of 8192^3 reaches 1157;
+// both hold the clock at 1.5-1.9 of 2.4 GHz, so power bounds them).
 constexpr int kTile = 64 * kC;          // values of a tile
 constexpr int kPhase = 16 * kC;         // ... of a phase
 constexpr int kChunk = 16 * 8;          // ... of a phase's channel chunk
@@ -176,9 +181,9 @@ __device__ inline u32x4 dpp4(u32x4 old, u32x4 src)
 }
 
 // Wavefronts per convolution work-group; the layer's weights (55 KB of LDS)
-// allow two work-groups per CU.  Four (two wavefronts per SIMD) measured
-// faster than six (three per SIMD): 539 against 451 TFLOP/s over the 18
-// layers of a 128x256x256 volume.
+// allow two work-groups per CU.  Over the 18 layers of 128x256x256 voxels, four
+// (two wavefronts per SIMD) took 8.23 ms and one work-group of eight per CU
+// 8.38; six (three per SIMD) were slower before (451 against 539 TFLOP/s).
 #ifndef DXG_CONV_WAVES
 #define DXG_CONV_WAVES 4
 #endif
@@ -224,8 +229,7 @@ struct RowsTile {
 // row y + 1 is stored when it exists.
 // The epilogue's configuration as template bits (EPI >= 0), so that a layer's
 // code holds only its own epilogue: the runtime tests of the residual, gate,
-// activation and output kind cost instructions (and branches) on every store,
-// and the wavefront's instruction fetch is what the convolution waits on.
+// activation and output kind cost instructions (and branches) on every store.
 // EPI < 0 reads the configuration from the arguments.
 constexpr int kEpiRelu = 1, kEpiRes = 2, kEpiGate = 4, kEpiY = 8, kEpiY32 = 16, kEpiY32All = 32;
 

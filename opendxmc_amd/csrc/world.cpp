@@ -16,6 +16,7 @@
 #include <memory>
 #include <map>
 #include <mutex>
+#include <shared_mutex>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -68,6 +69,29 @@ struct DevBuf {
 };
 
 }  // namespace
+
+// Turns at a world's scores, in the order asked for: a launch that adds to them
+// has them alone, reads share them.  A read takes many launches on the world's
+// stream, so without turns those of a run in another thread fall between them
+// and the arrays hold voxels of different moments.  The queue mutex keeps a run
+// of many launches from taking the next turn ahead of a read that waits.
+class ScoreTurns {
+public:
+    std::unique_lock<std::shared_mutex> change()
+    {
+        std::lock_guard<std::mutex> next(queue);
+        return std::unique_lock<std::shared_mutex>(scores);
+    }
+    std::shared_lock<std::shared_mutex> read() const
+    {
+        std::lock_guard<std::mutex> next(queue);
+        return std::shared_lock<std::shared_mutex>(scores);
+    }
+
+private:
+    mutable std::mutex queue;
+    mutable std::shared_mutex scores;
+};
 
 struct dxg_progress {
     std::atomic<uint64_t> n { 0 };
@@ -126,6 +150,7 @@ struct dxg_world {
     dxg_counters counters {};
     uint64_t generation = 0;   // world builds so far
     dxg::IoHold io;            // score reads
+    ScoreTurns turns;          // at the tally and the history count
 
     ~dxg_world()
     {
@@ -529,6 +554,7 @@ int dxg_world_clear_scores(dxg_world* w)
 {
     if (!w || !w->built)
         return fail(DXG_ERR_STATE, "dxg_world_clear_scores: world not built");
+    const auto turn = w->turns.change();
     HIP_TRY(hipMemsetAsync(w->d_tally.ptr, 0, w->tallyDoubles() * static_cast<size_t>(w->replicas) * sizeof(double), w->stream));
     HIP_TRY(hipStreamSynchronize(w->stream));
     w->histories = 0;
@@ -898,6 +924,7 @@ int runChunks(dxg_world* w, DevParams& p, uint64_t total, dxg_progress* progress
         const unsigned long long most = p.batch;   // put back below: later ranges may be longer
         if (!explicit_batch)
             p.batch = dxg::claimSize(h_end - h_begin, blocks, most);
+        const auto turn = w->turns.change();   // until the histories are counted
         dxg::launchReset(p.pool, p.counters, w->stream);
         const auto t0 = std::chrono::steady_clock::now();
         if (events)
@@ -1008,9 +1035,12 @@ int runChunks(dxg_world* w, DevParams& p, uint64_t total, dxg_progress* progress
         (void)hipEventDestroy(ev0);
         (void)hipEventDestroy(ev1);
     }
-    dxg::launchTallyFold(p.tally, p.tally_stride, p.tally_replicas, w->stream);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(w->stream));
+    {
+        const auto turn = w->turns.change();
+        dxg::launchTallyFold(p.tally, p.tally_stride, p.tally_replicas, w->stream);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(w->stream));
+    }
     acc.refill_threshold = p.refill_threshold;
     acc.interact_threshold = p.interact_threshold;
     acc.outer_threshold = p.outer_threshold;
@@ -1132,6 +1162,7 @@ int dxg_read_energy_scores(const dxg_world* w, double* sum_e, double* sum_e2, ui
 {
     if (!w || !w->built)
         return fail(DXG_ERR_STATE, "dxg_read_energy_scores: world not built");
+    const auto turn = w->turns.read();
     return readScores(w, sum_e != nullptr, sum_e2 != nullptr, n_events != nullptr,
                       [&](uint64_t v, uint64_t n, const double* e, const double* e2, const uint64_t* ev) {
                           if (sum_e)
@@ -1147,6 +1178,7 @@ int dxg_read_dose_scores(const dxg_world* w, double* dose_mgy, double* variance_
 {
     if (!w || !w->built)
         return fail(DXG_ERR_STATE, "dxg_read_dose_scores: world not built");
+    const auto turn = w->turns.read();
     const double voxel_cm3 = w->spacing[0] * w->spacing[1] * w->spacing[2];
     const double H = static_cast<double>(w->histories);
     return readScores(w, dose_mgy || variance_mgy2, variance_mgy2 != nullptr, n_events != nullptr,

@@ -6,6 +6,7 @@ from __future__ import annotations
 from concurrent.futures import ThreadPoolExecutor
 
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -76,6 +77,37 @@ def test_concurrent_reads():
     for k, r in zip(jobs, got):
         for a, b in zip(r, want[k]):
             np.testing.assert_array_equal(a, b)
+
+
+def test_read_during_runs_is_a_state_between_launches():
+    """Events read in one thread while another runs one launch after the other:
+    every read is the scores after some launch, none a mixture of several."""
+    world, grid, _ = scored_world((200, 181, 120), histories=20_000)   # one tally copy, 23 chunks a read
+    beam = dx.DXBeam({13: 2.0})
+    beam.setCollimation((20.0, 20.0))
+    beam.setNumberOfParticlesPerExposure(200_000)
+    states, stop = [grid.counters()["deposits"]], threading.Event()
+
+    def run():
+        tr = dx.Transport(seed=9)
+        for _ in range(2000):
+            if stop.is_set() or not tr(world, beam, None, False):
+                break
+            states.append(states[-1] + grid.counters()["deposits"])
+
+    thread = threading.Thread(target=run)
+    thread.start()
+    try:
+        reads = []
+        for _ in range(12):
+            ev = np.empty(grid.size(), dtype=np.uint64)
+            N.check(N.lib().dxg_read_energy_scores(grid._h, None, None, N.ptr(ev, N.u64)))
+            reads.append(int(ev.sum()))
+    finally:
+        stop.set()
+        thread.join()
+    assert reads[0] < reads[-1]
+    assert set(reads) <= set(states)
 
 
 @pytest.mark.parametrize("n", [1, (1 << 19) - 1, 1 << 19, 12 * 23168 + 1, 16 * 185024 + 5, 4_000_037])

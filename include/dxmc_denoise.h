@@ -46,14 +46,16 @@ int dxg_denoiser_get_grads(const dxg_denoiser* d, float* grads, uint64_t n);
 
 /* One Adam step (lr, beta1 0.9, beta2 0.999, eps 1e-8) on a batch of patches.
  * features: batch x D x H x W x 4 (float), target / mask: batch x D x H x W.
- * Loss = sum(mask (pred - target)^2) / sum(mask), written to *loss. */
+ * Loss = sum(mask (pred - target)^2) / sum(mask), written to *loss; a mask
+ * whose sum is not positive is refused and leaves the parameters as they were. */
 int dxg_denoiser_train_step(dxg_denoiser* d, const float* features, const float* target, const float* mask,
                             uint64_t batch, const uint64_t dims[3], float lr, float* loss);
 
 /* Prediction (relative dose) for one volume, host arrays; D x H x W. */
 int dxg_denoiser_infer(dxg_denoiser* d, const float* features, const uint64_t dims[3], float* prediction);
 
-/* Kernel timing of the last call (ms, HIP events). */
+/* Kernel timing of the last call (ms, HIP events); of a training step from its
+ * first copy to its last kernel, the copies and waits between them included. */
 double dxg_denoiser_last_ms(const dxg_denoiser* d);
 
 /* ---- on-device path from a built world after dxg_transport_run: nothing of

@@ -2089,6 +2089,14 @@ int dxg_denoiser_train_step(dxg_denoiser* d, const float* features, const float*
     if (!(lr > 0.0f) || !std::isfinite(lr))
         return fail(DXG_ERR_ARGUMENT, "dxg_denoiser_train_step: learning rate must be positive");
     const size_t nv = dm.voxels();
+    // The mask's sum is taken beside the forward pass; a mask without one positive
+    // value is refused here, where nothing is allocated or started yet.
+    if (std::none_of(mask, mask + nv, [](float v) { return v > 0.0f; }))
+        return fail(DXG_ERR_ARGUMENT, "dxg_denoiser_train_step: empty mask");
+    struct Settled {   // nothing of a step that fails runs on after it
+        hipStream_t stream;
+        ~Settled() { (void)hipStreamSynchronize(stream); }
+    } settled { d->stream };
     HIP_TRY(hipEventRecord(d->ev0, d->stream));
     if (int rc = d->upload(features, dm, true); rc != DXG_OK)
         return rc;

@@ -312,6 +312,31 @@ def test_network_loss_and_gradients_match_reference():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["zeros", "negative", "nan", "sum below zero", "one nan"])
+def test_refused_mask_changes_nothing(kind):
+    """A mask whose sum is not positive is an argument error; one without any
+    positive value is refused before anything is allocated (a step on these
+    patches takes 1.2 GB).  The next step is that of a fresh network."""
+    f, target, mask = _net_case(61, 4, (64, 64, 64))
+    refused = np.full_like(mask, {"zeros": 0.0, "negative": -1.0, "nan": np.nan, "sum below zero": -1.0}.get(kind, 1.0))
+    if kind == "sum below zero":
+        refused[0, 0] = 1.0
+    if kind == "one nan":
+        refused[-1, -1, -1, -1] = np.nan
+    net, fresh = dn.Denoiser(seed=7), dn.Denoiser(seed=7)
+    free = torch.cuda.mem_get_info()[0]
+    with pytest.raises(N.NativeError) as e:
+        net.train_step(f, target, refused, lr=1e-3)
+    assert e.value.code == N.DXG_ERR_ARGUMENT
+    if kind in ("zeros", "negative", "nan"):
+        assert free - torch.cuda.mem_get_info()[0] < 64 << 20
+    np.testing.assert_array_equal(net.params(), fresh.params())
+    assert net.train_step(f, target, mask, lr=1e-3) == fresh.train_step(f, target, mask, lr=1e-3)
+    np.testing.assert_array_equal(net.grads(), fresh.grads())
+    np.testing.assert_array_equal(net.params(), fresh.params())
+
+
+@pytest.mark.gpu
 def test_training_lowers_the_loss():
     """Noisy copies of a smooth dose field: the untrained network is the
     identity (loss = noise variance); training must remove part of the noise."""

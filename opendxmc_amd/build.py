@@ -84,17 +84,28 @@ def build_oracle() -> Path:
     return ORACLE_LIB
 
 
-HARNESS_SRC = ROOT / "tests" / "cpp" / "worker_harness.cpp"
-HARNESS = ROOT / "tests" / "cpp" / "_build" / "worker_harness"
+TESTS_CPP = ROOT / "tests" / "cpp"
+HARNESS = TESTS_CPP / "_build" / "worker_harness"
+PINNED_CHECK = TESTS_CPP / "_build" / "pinned_memory_check"
+
+
+def _build_program(out: Path, *extra: str) -> Path:
+    """A C++ program of tests/cpp on the library's C-ABI."""
+    out.parent.mkdir(parents=True, exist_ok=True)
+    _run(["g++", "-std=c++20", "-O2", "-Wall", "-Wextra", f"-I{ROOT / 'include'}", str(TESTS_CPP / f"{out.name}.cpp"),
+          f"-L{PKG}", "-ldxmc_hip", f"-Wl,-rpath,{PKG}", "-Wl,-rpath,$ORIGIN/../../../opendxmc_amd",
+          *extra, "-o", str(out)])
+    return out
 
 
 def build_harness() -> Path:
     """The C++ reproduction of the reference's worker<C>, on the C++ facade."""
-    HARNESS.parent.mkdir(parents=True, exist_ok=True)
-    _run(["g++", "-std=c++20", "-O2", "-Wall", "-Wextra", f"-I{ROOT / 'include'}", str(HARNESS_SRC),
-          f"-L{PKG}", "-ldxmc_hip", f"-Wl,-rpath,{PKG}", "-Wl,-rpath,$ORIGIN/../../../opendxmc_amd",
-          "-o", str(HARNESS)])
-    return HARNESS
+    return _build_program(HARNESS)
+
+
+def build_pinned_check() -> Path:
+    """Transfers with pinned allocations counted."""
+    return _build_program(PINNED_CHECK, "-ldl")
 
 
 def build_all() -> None:
@@ -102,6 +113,7 @@ def build_all() -> None:
     build_library()
     build_oracle()
     build_harness()
+    build_pinned_check()
 
 
 if __name__ == "__main__":

@@ -1669,12 +1669,12 @@ struct dxg_denoiser {
     // Bulk copies between host arrays and the device, complete on return.
     int toDevice(void* dst, const void* src, size_t bytes, hipStream_t on)
     {
-        HIP_TRY(dxg::ioUpload(on, dst, src, bytes));
+        HIP_TRY(dxg::ioUpload(io, on, dst, src, bytes));
         return DXG_OK;
     }
     int toHost(void* dst, const void* src, size_t bytes)
     {
-        HIP_TRY(dxg::ioDownload(stream, dst, src, bytes));
+        HIP_TRY(dxg::ioDownload(io, stream, dst, src, bytes));
         return DXG_OK;
     }
 

@@ -102,7 +102,7 @@ struct Lease {
 // The calling thread enqueues chunks as their slots are ready and polls the
 // oldest one's event; worker threads fill and drain.  With the runtime's calls
 // spread over the workers instead, 16 MB to the device took 1.3 ms (0.9 now).
-hipError_t ioRun(hipStream_t stream, size_t chunks, const IoHost& fill, const IoEnqueue& enqueue, const IoHost& drain)
+hipError_t ioRun(const IoHold&, hipStream_t stream, size_t chunks, const IoHost& fill, const IoEnqueue& enqueue, const IoHost& drain)
 {
     if (chunks == 0)
         return hipSuccess;
@@ -229,7 +229,7 @@ IoHold::~IoHold()
         delete s;
 }
 
-hipError_t ioUpload(hipStream_t stream, void* dst, const void* src, size_t bytes)
+hipError_t ioUpload(const IoHold& hold, hipStream_t stream, void* dst, const void* src, size_t bytes)
 {
     if (bytes < kIoUploadLeast) {
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
@@ -238,11 +238,11 @@ hipError_t ioUpload(hipStream_t stream, void* dst, const void* src, size_t bytes
     const size_t per = ioChunk(bytes, 1, 4096);
     auto size = [&](size_t i) { return std::min(per, bytes - i * per); };
     return ioRun(
-        stream, (bytes + per - 1) / per, [&](size_t i, char* slot) { std::memcpy(slot, static_cast<const char*>(src) + i * per, size(i)); },
+        hold, stream, (bytes + per - 1) / per, [&](size_t i, char* slot) { std::memcpy(slot, static_cast<const char*>(src) + i * per, size(i)); },
         [&](size_t i, char* slot) { return hipMemcpyAsync(static_cast<char*>(dst) + i * per, slot, size(i), hipMemcpyHostToDevice, stream); }, nullptr);
 }
 
-hipError_t ioDownload(hipStream_t stream, void* dst, const void* src, size_t bytes)
+hipError_t ioDownload(const IoHold& hold, hipStream_t stream, void* dst, const void* src, size_t bytes)
 {
     if (bytes < kIoDownloadLeast) {
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
@@ -251,7 +251,7 @@ hipError_t ioDownload(hipStream_t stream, void* dst, const void* src, size_t byt
     const size_t per = ioChunk(bytes, 1, 4096);
     auto size = [&](size_t i) { return std::min(per, bytes - i * per); };
     return ioRun(
-        stream, (bytes + per - 1) / per, nullptr,
+        hold, stream, (bytes + per - 1) / per, nullptr,
         [&](size_t i, char* slot) { return hipMemcpyAsync(slot, static_cast<const char*>(src) + i * per, size(i), hipMemcpyDeviceToHost, stream); },
         [&](size_t i, char* slot) { std::memcpy(static_cast<char*>(dst) + i * per, slot, size(i)); });
 }

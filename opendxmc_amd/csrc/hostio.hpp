@@ -18,6 +18,19 @@ constexpr int kIoThreads = 12;
 constexpr int kIoSlots = 16;
 constexpr size_t kIoSlotBytes = size_t(3) << 20;
 
+// The pinned slots come from at most kIoIdle idle sets kept for the next call
+// (allocating and freeing one takes 0.4 ms); they are freed when the last one
+// that holds them is gone: worlds, denoisers, and threads that called the
+// segmentation or the dose table with host arrays.  Every transfer names the
+// hold it runs under: without one, it would allocate and free a set.
+constexpr int kIoIdle = 2;
+struct IoHold {
+    IoHold();
+    ~IoHold();
+    IoHold(const IoHold&) = delete;
+    IoHold& operator=(const IoHold&) = delete;
+};
+
 // Runs a transfer in chunks: fill(i, slot) puts host data of chunk i into its
 // slot, enqueue(i, slot) puts the device work on `stream` that uses the slot
 // (slots are device-accessible), drain(i, slot) takes results into host arrays.
@@ -26,26 +39,14 @@ constexpr size_t kIoSlotBytes = size_t(3) << 20;
 // every chunk is through; the first error ends it.
 using IoEnqueue = std::function<hipError_t(size_t chunk, char* slot)>;
 using IoHost = std::function<void(size_t chunk, char* slot)>;
-hipError_t ioRun(hipStream_t stream, size_t chunks, const IoHost& fill, const IoEnqueue& enqueue, const IoHost& drain);
+hipError_t ioRun(const IoHold& hold, hipStream_t stream, size_t chunks, const IoHost& fill, const IoEnqueue& enqueue, const IoHost& drain);
 
 // Copies `bytes` to or from device memory, complete on return.  Short ones go
 // straight to the runtime's own copy (29 GB/s to the device and 17 GB/s back,
 // less on fresh pages): starting the threads costs 0.2 ms.
-hipError_t ioUpload(hipStream_t stream, void* dst, const void* src, size_t bytes);
-hipError_t ioDownload(hipStream_t stream, void* dst, const void* src, size_t bytes);
+hipError_t ioUpload(const IoHold& hold, hipStream_t stream, void* dst, const void* src, size_t bytes);
+hipError_t ioDownload(const IoHold& hold, hipStream_t stream, void* dst, const void* src, size_t bytes);
 constexpr size_t kIoUploadLeast = size_t(24) << 20, kIoDownloadLeast = size_t(3) << 20;
-
-// The pinned slots come from at most kIoIdle idle sets kept for the next call
-// (allocating and freeing one takes 0.4 ms); they are freed when the last one
-// that holds them is gone: worlds, denoisers, and threads that called the
-// segmentation or the dose table with host arrays.
-constexpr int kIoIdle = 2;
-struct IoHold {
-    IoHold();
-    ~IoHold();
-    IoHold(const IoHold&) = delete;
-    IoHold& operator=(const IoHold&) = delete;
-};
 
 // Items of a chunk: about two chunks a thread for a small transfer, at most what
 // a slot holds; a multiple of `multiple`.

@@ -469,6 +469,13 @@ int runSegmentation(const dxg_ct_segmentation& t, const double* hu, uint64_t n, 
     return tm.stop(s, g_last_ms[0]);
 }
 
+// The calling thread's hold on the pinned slots.
+const dxg::IoHold& threadHold()
+{
+    thread_local dxg::IoHold io;
+    return io;
+}
+
 constexpr uint64_t kSegHostLeast = 1u << 19;
 
 // Host arrays: the kernel reads CT numbers from pinned slots and writes its
@@ -479,7 +486,6 @@ constexpr uint64_t kSegHostLeast = 1u << 19;
 // carries 8 bytes a voxel in and 9 out.
 int segmentHost(const dxg_ct_segmentation& t, const double* hu, uint64_t n, uint8_t* mat, double* dens)
 {
-    thread_local dxg::IoHold io;
     const SegArgs a = segArgs(t);
     const uint64_t per = dxg::ioChunk(n, 17, 64);
     auto size = [&](size_t c) { return std::min(per, n - c * per); };
@@ -491,7 +497,7 @@ int segmentHost(const dxg_ct_segmentation& t, const double* hu, uint64_t n, uint
     if (rc = tm.start(nullptr); rc != DXG_OK)
         return rc;
     const hipError_t e = dxg::ioRun(
-        nullptr, (n + per - 1) / per, [&](size_t c, char* slot) { std::memcpy(slot, hu + c * per, size(c) * sizeof(double)); },
+        threadHold(), nullptr, (n + per - 1) / per, [&](size_t c, char* slot) { std::memcpy(slot, hu + c * per, size(c) * sizeof(double)); },
         [&](size_t c, char* slot) {
             rc = launchSegmentation(a, reinterpret_cast<const double*>(slot), size(c), matAt(slot), densAt(slot), nullptr);
             return rc == DXG_OK ? hipSuccess : hipErrorUnknown;
@@ -692,11 +698,11 @@ int dxg_ct_segment(const dxg_ct_segmentation* t, const double* hu, uint64_t n, u
         return rc;
     if (int rc = dm.alloc(n); rc != DXG_OK)
         return rc;
-    HIP_TRY(dxg::ioUpload(nullptr, dh.p, hu, n * sizeof(double)));
+    HIP_TRY(dxg::ioUpload(threadHold(), nullptr, dh.p, hu, n * sizeof(double)));
     if (int rc = runSegmentation(*t, dh.p, n, dm.p, dd.p, nullptr); rc != DXG_OK)
         return rc;
-    HIP_TRY(dxg::ioDownload(nullptr, material, dm.p, n));
-    HIP_TRY(dxg::ioDownload(nullptr, density, dd.p, n * sizeof(double)));
+    HIP_TRY(dxg::ioDownload(threadHold(), nullptr, material, dm.p, n));
+    HIP_TRY(dxg::ioDownload(threadHold(), nullptr, density, dd.p, n * sizeof(double)));
     return DXG_OK;
 }
 
@@ -729,7 +735,6 @@ int dxg_organ_dose_table(const uint8_t* organ, const double* dose, const double*
     }
     if (!organ || !dose || !density)
         return fail(DXG_ERR_ARGUMENT, "dxg_organ_dose_table: null argument");
-    thread_local dxg::IoHold io;
     DeviceBuffer<uint8_t> dorg;
     DeviceBuffer<double> ddose, ddens;
     if (int rc = dorg.alloc(n); rc != DXG_OK)
@@ -738,9 +743,9 @@ int dxg_organ_dose_table(const uint8_t* organ, const double* dose, const double*
         return rc;
     if (int rc = ddens.alloc(n); rc != DXG_OK)
         return rc;
-    HIP_TRY(dxg::ioUpload(nullptr, dorg.p, organ, n));
-    HIP_TRY(dxg::ioUpload(nullptr, ddose.p, dose, n * sizeof(double)));
-    HIP_TRY(dxg::ioUpload(nullptr, ddens.p, density, n * sizeof(double)));
+    HIP_TRY(dxg::ioUpload(threadHold(), nullptr, dorg.p, organ, n));
+    HIP_TRY(dxg::ioUpload(threadHold(), nullptr, ddose.p, dose, n * sizeof(double)));
+    HIP_TRY(dxg::ioUpload(threadHold(), nullptr, ddens.p, density, n * sizeof(double)));
     return runTable(dorg.p, ddose.p, ddens.p, n, spacing_cm, out, nullptr);
 }
 

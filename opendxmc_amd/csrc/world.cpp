@@ -1095,7 +1095,7 @@ int readScores(const dxg_world* w, bool want_e, bool want_e2, bool want_events, 
     int before = 0;   // the caller's current device, put back below
     HIP_TRY(hipGetDevice(&before));
     HIP_TRY(hipSetDevice(w->device));
-    const hipError_t status = dxg::ioRun(w->stream, (n + per - 1) / per, nullptr, enqueue, drain);
+    const hipError_t status = dxg::ioRun(w->io, w->stream, (n + per - 1) / per, nullptr, enqueue, drain);
     HIP_TRY(hipSetDevice(before));
     HIP_TRY(status);
     return DXG_OK;

@@ -6,6 +6,7 @@ from __future__ import annotations
 from concurrent.futures import ThreadPoolExecutor
 
 import ctypes as C
+import subprocess
 import threading
 
 import numpy as np
@@ -13,6 +14,7 @@ import pytest
 
 import opendxmc_amd as dx
 from opendxmc_amd import _native as N
+from opendxmc_amd import build
 from opendxmc_amd import phantoms
 from opendxmc_amd import pipelines as P
 from opendxmc_amd.devmem import DeviceBuffer
@@ -139,3 +141,12 @@ def test_dose_table_of_large_host_arrays_equals_resident():
     bufs = [DeviceBuffer.from_array(a) for a in (organ, dose, dens)]
     dev = P.organ_dose_table_device(bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, n, (0.1, 0.1, 0.1))
     np.testing.assert_array_equal(P.organ_dose_table(organ, dose, dens, (0.1, 0.1, 0.1)), dev)
+
+
+@pytest.mark.parametrize("case", ["held"])
+def test_pinned_memory(case):
+    """tests/cpp/pinned_memory_check.cpp, whose own hipHostMalloc the library calls."""
+    if not build.PINNED_CHECK.exists():
+        build.build_pinned_check()
+    r = subprocess.run([str(build.PINNED_CHECK), case], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr

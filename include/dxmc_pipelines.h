@@ -82,7 +82,7 @@ int dxg_organ_dose_table_device(const uint8_t* organ, const double* dose, const 
 
 /* Mean duration (ms) of the last launch of each kernel on this thread, from
  * HIP events around it on its stream: which = 0 segmentation (from host arrays
- * of 2^19 voxels and more: all of its launches and the transfers between
+ * of 393,216 voxels and more: all of its launches and the transfers between
  * them), 1 dose table (both of its kernels). */
 double dxg_pipeline_last_ms(int which);
 

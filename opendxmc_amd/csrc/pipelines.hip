@@ -476,7 +476,12 @@ const dxg::IoHold& threadHold()
     return io;
 }
 
-constexpr uint64_t kSegHostLeast = 1u << 19;
+// Voxels from which host arrays go through the slots: where the densities of the
+// other path, whole arrays in device buffers, would take the slots on their way
+// back.  Slots / device buffers, us a call, in a process of its own: 262,144
+// voxels 300-330 / 302, 393,000 372-396 / 380, 430,000 397-417 / 562, 524,288
+// 447-474 / 613-639, 1,048,576 597-622 / 1004-1044.
+constexpr uint64_t kSegHostLeast = dxg::kIoDownloadLeast / sizeof(double);
 
 // Host arrays: the kernel reads CT numbers from pinned slots and writes its
 // results into them, chunk by chunk, while host threads fill and drain others,
@@ -684,10 +689,8 @@ int dxg_ct_segment(const dxg_ct_segmentation* t, const double* hu, uint64_t n, u
         return DXG_OK;
     if (!hu || !material || !density)
         return fail(DXG_ERR_ARGUMENT, "dxg_ct_segment: null argument");
-    // through slots, except that starting threads costs a small volume more than
-    // three device buffers do (260,000 voxels: 0.88 against 0.76 ms a call, equal
-    // at 500,000), and that outputs over the input may be written only after all
-    // of it was read
+    // through slots, except that small volumes gain nothing by it and that outputs
+    // over the input may be written only after all of it was read
     if (n >= kSegHostLeast && !overlap(hu, n * sizeof(double), material, n) && !overlap(hu, n * sizeof(double), density, n * sizeof(double)))
         return segmentHost(*t, hu, n, material, density);
     DeviceBuffer<double> dh, dd;

@@ -1,10 +1,13 @@
 // Transfers of the library against its pinned slots, seen through this
-// program's own hipHostMalloc, which the library binds to: it counts the calls
-// and passes them on.
+// program's own hipHostMalloc and hipMalloc, which the library binds to: they
+// count the calls and pass them on.
 //
-// usage: pinned_memory_check held
-// held: two segmentations of a volume that goes through device buffers, in a
-//       process where nothing else holds slots, allocate one set of slots.
+// usage: pinned_memory_check held | segment
+// held: two segmentations that go through device buffers (the densities replace
+//       the CT numbers), in a process where nothing else holds slots, allocate
+//       one set of slots.
+// segment: host arrays of 393,216 voxels go through slots, fewer through three
+//          device buffers.
 #include "dxmc_pipelines.h"
 
 #include <dlfcn.h>
@@ -17,7 +20,7 @@
 
 namespace {
 
-int g_allocations = 0;
+int g_allocations = 0, g_device_allocations = 0;
 
 int failed(const char* what)
 {
@@ -51,14 +54,30 @@ int held()
 {
     const dxg_ct_segmentation t = threeMaterials();
     const std::size_t n = 500'000;
-    const std::vector<double> hu = ctNumbers(n);
+    std::vector<double> hu = ctNumbers(n);
     std::vector<std::uint8_t> material(n);
-    std::vector<double> density(n);
     for (int call = 0; call < 2; ++call)
-        if (dxg_ct_segment(&t, hu.data(), n, material.data(), density.data()) != DXG_OK)
+        if (dxg_ct_segment(&t, hu.data(), n, material.data(), hu.data()) != DXG_OK)
             return failed("dxg_ct_segment");
     std::printf("%d allocations\n", g_allocations);
     return g_allocations == 1 ? 0 : 2;
+}
+
+int segment()
+{
+    const dxg_ct_segmentation t = threeMaterials();
+    const std::size_t most = 393'216;
+    const std::vector<double> hu = ctNumbers(most);
+    std::vector<std::uint8_t> material(most);
+    std::vector<double> density(most);
+    for (std::size_t n : { most - 1, most }) {
+        if (dxg_ct_segment(&t, hu.data(), n, material.data(), density.data()) != DXG_OK)
+            return failed("dxg_ct_segment");
+        std::printf("%zu voxels: %d pinned, %d device allocations so far\n", n, g_allocations, g_device_allocations);
+        if (g_allocations != (n < most ? 0 : 1) || g_device_allocations != 3)
+            return 2;
+    }
+    return 0;
 }
 
 }  // namespace
@@ -70,10 +89,19 @@ extern "C" int hipHostMalloc(void** p, std::size_t bytes, unsigned flags)
     return real(p, bytes, flags);
 }
 
+extern "C" int hipMalloc(void** p, std::size_t bytes)
+{
+    static const auto real = reinterpret_cast<int (*)(void**, std::size_t)>(dlsym(RTLD_NEXT, "hipMalloc"));
+    ++g_device_allocations;
+    return real(p, bytes);
+}
+
 int main(int argc, char** argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "held")
         return held();
+    if (what == "segment")
+        return segment();
     return 64;
 }

@@ -112,10 +112,10 @@ def test_read_during_runs_is_a_state_between_launches():
     assert set(reads) <= set(states)
 
 
-@pytest.mark.parametrize("n", [1, (1 << 19) - 1, 1 << 19, 12 * 23168 + 1, 16 * 185024 + 5, 4_000_037])
+@pytest.mark.parametrize("n", [1, 393_215, 393_216, (1 << 19) - 1, 1 << 19, 12 * 23168 + 1, 16 * 185024 + 5, 4_000_037])
 def test_segmentation_of_host_arrays_equals_resident(n):
-    """The same bits whichever way the voxels travel, up to 2^19 voxels through
-    whole device buffers and above in chunks; with the densities over the CT
+    """The same bits whichever way the voxels travel, below 393,216 voxels through
+    whole device buffers and from there in chunks; with the densities over the CT
     numbers too."""
     rng = np.random.default_rng(n)
     hu = rng.uniform(-1100.0, 2500.0, n)
@@ -143,7 +143,7 @@ def test_dose_table_of_large_host_arrays_equals_resident():
     np.testing.assert_array_equal(P.organ_dose_table(organ, dose, dens, (0.1, 0.1, 0.1)), dev)
 
 
-@pytest.mark.parametrize("case", ["held"])
+@pytest.mark.parametrize("case", ["held", "segment"])
 def test_pinned_memory(case):
     """tests/cpp/pinned_memory_check.cpp, whose own hipHostMalloc the library calls."""
     if not build.PINNED_CHECK.exists():

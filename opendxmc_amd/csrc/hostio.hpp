@@ -42,11 +42,14 @@ using IoHost = std::function<void(size_t chunk, char* slot)>;
 hipError_t ioRun(const IoHold& hold, hipStream_t stream, size_t chunks, const IoHost& fill, const IoEnqueue& enqueue, const IoHost& drain);
 
 // Copies `bytes` to or from device memory, complete on return.  Short ones go
-// straight to the runtime's own copy (29 GB/s to the device and 17 GB/s back,
-// less on fresh pages): starting the threads costs 0.2 ms.
+// straight to the runtime's own copy: starting the threads costs 0.2 ms.  Runtime
+// / slots, us, medians of two processes: up 24 MB 685 / 1050, 32 MB 930-1060 /
+// 1220-1310, 40 MB 1280-1580 / 1390-1510, 44 MB 1460-1780 / 1470-1730, 48 MB
+// 1610-1970 / 1540-1690, 64 MB 2200-2540 / 1850-2040; down 1 MB into warm pages 67
+// / 77 and fresh ones 240 / 170, 3 MB 205 / 217 and 745-820 / 360-425.
 hipError_t ioUpload(const IoHold& hold, hipStream_t stream, void* dst, const void* src, size_t bytes);
 hipError_t ioDownload(const IoHold& hold, hipStream_t stream, void* dst, const void* src, size_t bytes);
-constexpr size_t kIoUploadLeast = size_t(24) << 20, kIoDownloadLeast = size_t(3) << 20;
+constexpr size_t kIoUploadLeast = size_t(44) << 20, kIoDownloadLeast = size_t(3) << 20;
 
 // Items of a chunk: about two chunks a thread for a small transfer, at most what
 // a slot holds; a multiple of `multiple`.

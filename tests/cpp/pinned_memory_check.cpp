@@ -2,12 +2,13 @@
 // program's own hipHostMalloc and hipMalloc, which the library binds to: they
 // count the calls and pass them on.
 //
-// usage: pinned_memory_check held | segment
+// usage: pinned_memory_check held | segment | upload
 // held: two segmentations that go through device buffers (the densities replace
 //       the CT numbers), in a process where nothing else holds slots, allocate
 //       one set of slots.
 // segment: host arrays of 393,216 voxels go through slots, fewer through three
 //          device buffers.
+// upload: the dose table's host arrays take slots from 44 MiB on.
 #include "dxmc_pipelines.h"
 
 #include <dlfcn.h>
@@ -80,6 +81,23 @@ int segment()
     return 0;
 }
 
+int upload()
+{
+    const std::size_t most = (std::size_t(44) << 20) / sizeof(double);
+    const std::vector<double> values(most, 1.0);
+    const std::vector<std::uint8_t> organ(most, 3);
+    const double spacing[3] = { 0.1, 0.1, 0.1 };
+    dxg_organ_dose rows[256];
+    for (std::size_t n : { most - 1, most }) {
+        if (dxg_organ_dose_table(organ.data(), values.data(), values.data(), n, spacing, rows) != DXG_OK)
+            return failed("dxg_organ_dose_table");
+        std::printf("%zu voxels: %d pinned allocations so far\n", n, g_allocations);
+        if (g_allocations != (n < most ? 0 : 1) || rows[3].n_voxels != n)
+            return 2;
+    }
+    return 0;
+}
+
 }  // namespace
 
 extern "C" int hipHostMalloc(void** p, std::size_t bytes, unsigned flags)
@@ -103,5 +121,7 @@ int main(int argc, char** argv)
         return held();
     if (what == "segment")
         return segment();
+    if (what == "upload")
+        return upload();
     return 64;
 }

@@ -133,8 +133,9 @@ def test_segmentation_of_host_arrays_equals_resident(n):
     assert P.last_ms(0) > 0.0
 
 
-def test_dose_table_of_large_host_arrays_equals_resident():
-    n = 4_500_001      # its 36 MB arrays go in chunks, the organ bytes in one piece
+# the 48 MB arrays of 6,000,001 voxels go in chunks, their organ bytes in one piece
+@pytest.mark.parametrize("n", [4_500_001, 6_000_001])
+def test_dose_table_of_large_host_arrays_equals_resident(n):
     rng = np.random.default_rng(5)
     organ = np.repeat(rng.integers(0, 256, n // 50 + 1, dtype=np.uint8), 50)[:n]
     dose, dens = rng.random(n), rng.uniform(0.0, 2.0, n)
@@ -143,7 +144,7 @@ def test_dose_table_of_large_host_arrays_equals_resident():
     np.testing.assert_array_equal(P.organ_dose_table(organ, dose, dens, (0.1, 0.1, 0.1)), dev)
 
 
-@pytest.mark.parametrize("case", ["held", "segment"])
+@pytest.mark.parametrize("case", ["held", "segment", "upload"])
 def test_pinned_memory(case):
     """tests/cpp/pinned_memory_check.cpp, whose own hipHostMalloc the library calls."""
     if not build.PINNED_CHECK.exists():

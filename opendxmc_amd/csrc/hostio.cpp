@@ -5,6 +5,7 @@
 #include <atomic>
 #include <cstring>
 #include <exception>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <thread>
@@ -86,30 +87,59 @@ struct Lease {
         }
         delete set;
     }
-    hipError_t prepare()
+    // The set, or null where the system has no more pinned memory to give (the
+    // refusal is cleared, so that no later check takes it for its own error).
+    const SlotSet* prepare()
     {
         int dev = 0;
-        if (const hipError_t e = hipGetDevice(&dev); e != hipSuccess)
-            return e;
         if (!set)
             set = new (std::nothrow) SlotSet;
-        return set ? set->prepare(dev) : hipErrorOutOfMemory;
+        if (set && hipGetDevice(&dev) == hipSuccess && set->prepare(dev) == hipSuccess)
+            return set;
+        (void)hipGetLastError();
+        delete set;
+        return set = nullptr;
     }
 };
 
-}  // namespace
+// A transfer without pinned slots: chunk after chunk through one piece of device
+// memory and one of pageable memory.
+hipError_t runUnpinned(hipStream_t stream, size_t chunks, const IoHost& fill, const IoEnqueue& enqueue, const IoHost& drain)
+{
+    struct DeviceSlot {
+        void* p = nullptr;
+        ~DeviceSlot()
+        {
+            if (p)
+                (void)hipFree(p);
+        }
+    } slot;
+    const std::unique_ptr<char[]> host(new (std::nothrow) char[kIoSlotBytes]());
+    if (!host)
+        return hipErrorOutOfMemory;
+    hipError_t e = hipMalloc(&slot.p, kIoSlotBytes);
+    for (size_t c = 0; c < chunks && e == hipSuccess; ++c) {
+        if (fill) {
+            fill(c, host.get());
+            e = hipMemcpyAsync(slot.p, host.get(), kIoSlotBytes, hipMemcpyHostToDevice, stream);
+        }
+        if (e == hipSuccess)
+            e = enqueue(c, static_cast<char*>(slot.p));
+        if (e == hipSuccess && drain)
+            e = hipMemcpyAsync(host.get(), slot.p, kIoSlotBytes, hipMemcpyDeviceToHost, stream);
+        if (const hipError_t done = hipStreamSynchronize(stream); e == hipSuccess)
+            e = done;
+        if (e == hipSuccess && drain)
+            drain(c, host.get());
+    }
+    return e;
+}
 
 // The calling thread enqueues chunks as their slots are ready and polls the
 // oldest one's event; worker threads fill and drain.  With the runtime's calls
 // spread over the workers instead, 16 MB to the device took 1.3 ms (0.9 now).
-hipError_t ioRun(const IoHold&, hipStream_t stream, size_t chunks, const IoHost& fill, const IoEnqueue& enqueue, const IoHost& drain)
+hipError_t run(const SlotSet& set, hipStream_t stream, size_t chunks, const IoHost& fill, const IoEnqueue& enqueue, const IoHost& drain)
 {
-    if (chunks == 0)
-        return hipSuccess;
-    Lease lease;
-    if (const hipError_t e = lease.prepare(); e != hipSuccess)
-        return e;
-    const SlotSet& set = *lease.set;
     if (chunks == 1) {   // no thread is worth starting
         if (fill)
             fill(0, set.p);
@@ -211,6 +241,23 @@ hipError_t ioRun(const IoHold&, hipStream_t stream, size_t chunks, const IoHost&
     return status;
 }
 
+hipError_t copyPageable(hipStream_t stream, void* dst, const void* src, size_t bytes, hipMemcpyKind kind)
+{
+    const hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, stream);
+    return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+}
+
+}  // namespace
+
+hipError_t ioRun(const IoHold&, hipStream_t stream, size_t chunks, const IoHost& fill, const IoEnqueue& enqueue, const IoHost& drain)
+{
+    if (chunks == 0)
+        return hipSuccess;
+    Lease lease;
+    const SlotSet* set = lease.prepare();
+    return set ? run(*set, stream, chunks, fill, enqueue, drain) : runUnpinned(stream, chunks, fill, enqueue, drain);
+}
+
 IoHold::IoHold()
 {
     std::lock_guard<std::mutex> lock(pool().mu);
@@ -229,31 +276,35 @@ IoHold::~IoHold()
         delete s;
 }
 
-hipError_t ioUpload(const IoHold& hold, hipStream_t stream, void* dst, const void* src, size_t bytes)
+hipError_t ioUpload(const IoHold&, hipStream_t stream, void* dst, const void* src, size_t bytes)
 {
-    if (bytes < kIoUploadLeast) {
-        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
-        return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+    if (bytes >= kIoUploadLeast) {
+        Lease lease;
+        const size_t per = ioChunk(bytes, 1, 4096);
+        auto size = [&](size_t i) { return std::min(per, bytes - i * per); };
+        if (const SlotSet* set = lease.prepare())
+            return run(
+                *set, stream, (bytes + per - 1) / per,
+                [&](size_t i, char* slot) { std::memcpy(slot, static_cast<const char*>(src) + i * per, size(i)); },
+                [&](size_t i, char* slot) { return hipMemcpyAsync(static_cast<char*>(dst) + i * per, slot, size(i), hipMemcpyHostToDevice, stream); },
+                nullptr);
     }
-    const size_t per = ioChunk(bytes, 1, 4096);
-    auto size = [&](size_t i) { return std::min(per, bytes - i * per); };
-    return ioRun(
-        hold, stream, (bytes + per - 1) / per, [&](size_t i, char* slot) { std::memcpy(slot, static_cast<const char*>(src) + i * per, size(i)); },
-        [&](size_t i, char* slot) { return hipMemcpyAsync(static_cast<char*>(dst) + i * per, slot, size(i), hipMemcpyHostToDevice, stream); }, nullptr);
+    return copyPageable(stream, dst, src, bytes, hipMemcpyHostToDevice);
 }
 
-hipError_t ioDownload(const IoHold& hold, hipStream_t stream, void* dst, const void* src, size_t bytes)
+hipError_t ioDownload(const IoHold&, hipStream_t stream, void* dst, const void* src, size_t bytes)
 {
-    if (bytes < kIoDownloadLeast) {
-        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
-        return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+    if (bytes >= kIoDownloadLeast) {
+        Lease lease;
+        const size_t per = ioChunk(bytes, 1, 4096);
+        auto size = [&](size_t i) { return std::min(per, bytes - i * per); };
+        if (const SlotSet* set = lease.prepare())
+            return run(
+                *set, stream, (bytes + per - 1) / per, nullptr,
+                [&](size_t i, char* slot) { return hipMemcpyAsync(slot, static_cast<const char*>(src) + i * per, size(i), hipMemcpyDeviceToHost, stream); },
+                [&](size_t i, char* slot) { std::memcpy(static_cast<char*>(dst) + i * per, slot, size(i)); });
     }
-    const size_t per = ioChunk(bytes, 1, 4096);
-    auto size = [&](size_t i) { return std::min(per, bytes - i * per); };
-    return ioRun(
-        hold, stream, (bytes + per - 1) / per, nullptr,
-        [&](size_t i, char* slot) { return hipMemcpyAsync(slot, static_cast<const char*>(src) + i * per, size(i), hipMemcpyDeviceToHost, stream); },
-        [&](size_t i, char* slot) { std::memcpy(static_cast<char*>(dst) + i * per, slot, size(i)); });
+    return copyPageable(stream, dst, src, bytes, hipMemcpyDeviceToHost);
 }
 
 }  // namespace dxg

@@ -34,6 +34,8 @@ struct IoHold {
 // Runs a transfer in chunks: fill(i, slot) puts host data of chunk i into its
 // slot, enqueue(i, slot) puts the device work on `stream` that uses the slot
 // (slots are device-accessible), drain(i, slot) takes results into host arrays.
+// Where pinned memory is refused the chunks pass one after another through 3 MB
+// of device memory and of pageable memory instead.
 // fill and drain run in several threads and may be empty; enqueue, like every
 // call of the runtime, runs in the caller's thread, in order.  Returns when
 // every chunk is through; the first error ends it.
@@ -41,8 +43,8 @@ using IoEnqueue = std::function<hipError_t(size_t chunk, char* slot)>;
 using IoHost = std::function<void(size_t chunk, char* slot)>;
 hipError_t ioRun(const IoHold& hold, hipStream_t stream, size_t chunks, const IoHost& fill, const IoEnqueue& enqueue, const IoHost& drain);
 
-// Copies `bytes` to or from device memory, complete on return.  Short ones go
-// straight to the runtime's own copy: starting the threads costs 0.2 ms.  Runtime
+// Copies `bytes` to or from device memory, complete on return.  Short ones, and
+// any where pinned memory is refused, go straight to the runtime's own copy: starting the threads costs 0.2 ms.  Runtime
 // / slots, us, medians of two processes: up 24 MB 685 / 1050, 32 MB 930-1060 /
 // 1220-1310, 40 MB 1280-1580 / 1390-1510, 44 MB 1460-1780 / 1470-1730, 48 MB
 // 1610-1970 / 1540-1690, 64 MB 2200-2540 / 1850-2040; down 1 MB into warm pages 67

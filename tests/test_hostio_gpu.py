@@ -144,7 +144,7 @@ def test_dose_table_of_large_host_arrays_equals_resident(n):
     np.testing.assert_array_equal(P.organ_dose_table(organ, dose, dens, (0.1, 0.1, 0.1)), dev)
 
 
-@pytest.mark.parametrize("case", ["held", "segment", "upload"])
+@pytest.mark.parametrize("case", ["held", "segment", "upload", "refused"])
 def test_pinned_memory(case):
     """tests/cpp/pinned_memory_check.cpp, whose own hipHostMalloc the library calls."""
     if not build.PINNED_CHECK.exists():

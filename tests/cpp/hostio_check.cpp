@@ -237,6 +237,9 @@ int main(int argc, char** argv)
         CHECK(g_last_error == hipSuccess);   // the next launch check must not report it
         g_refuse_pinned = false;
         everything();
+    } else if (what == "threads refused") {
+        g_refuse_threads = true;
+        everything();
     } else {
         return 64;
     }

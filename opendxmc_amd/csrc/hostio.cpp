@@ -67,6 +67,30 @@ Pool& pool()
     return *p;
 }
 
+// Makes a stream's device the current one for the length of a transfer: the
+// events recorded on the stream have to be of its device, whatever device the
+// calling thread is on.
+struct StreamDevice {
+    int device = 0, before = -1;   // before: to go back to, if another
+    hipError_t status;
+    explicit StreamDevice(hipStream_t stream)
+        : status(hipGetDevice(&device))
+    {
+        int own = device;
+        if (status == hipSuccess && stream)
+            status = hipStreamGetDevice(stream, &own);
+        if (status == hipSuccess && own != device && (status = hipSetDevice(own)) == hipSuccess) {
+            before = device;
+            device = own;
+        }
+    }
+    ~StreamDevice()
+    {
+        if (before >= 0)
+            (void)hipSetDevice(before);
+    }
+};
+
 // A set for one call, from the pool or new, put back or freed at its end.
 struct Lease {
     SlotSet* set = nullptr;
@@ -89,12 +113,11 @@ struct Lease {
     }
     // The set, or null where the system has no more pinned memory to give (the
     // refusal is cleared, so that no later check takes it for its own error).
-    const SlotSet* prepare()
+    const SlotSet* prepare(const StreamDevice& at)
     {
-        int dev = 0;
         if (!set)
             set = new (std::nothrow) SlotSet;
-        if (set && hipGetDevice(&dev) == hipSuccess && set->prepare(dev) == hipSuccess)
+        if (set && set->prepare(at.device) == hipSuccess)
             return set;
         (void)hipGetLastError();
         delete set;
@@ -266,8 +289,11 @@ hipError_t ioRun(const IoHold&, hipStream_t stream, size_t chunks, const IoHost&
 {
     if (chunks == 0)
         return hipSuccess;
+    const StreamDevice at(stream);
+    if (at.status != hipSuccess)
+        return at.status;
     Lease lease;
-    const SlotSet* set = lease.prepare();
+    const SlotSet* set = lease.prepare(at);
     return set ? run(*set, stream, chunks, fill, enqueue, drain) : runUnpinned(stream, chunks, fill, enqueue, drain);
 }
 
@@ -292,10 +318,11 @@ IoHold::~IoHold()
 hipError_t ioUpload(const IoHold&, hipStream_t stream, void* dst, const void* src, size_t bytes)
 {
     if (bytes >= kIoUploadLeast) {
+        const StreamDevice at(stream);
         Lease lease;
         const size_t per = ioChunk(bytes, 1, 4096);
         auto size = [&](size_t i) { return std::min(per, bytes - i * per); };
-        if (const SlotSet* set = lease.prepare())
+        if (const SlotSet* set = at.status == hipSuccess ? lease.prepare(at) : nullptr)
             return run(
                 *set, stream, (bytes + per - 1) / per,
                 [&](size_t i, char* slot) { std::memcpy(slot, static_cast<const char*>(src) + i * per, size(i)); },
@@ -308,10 +335,11 @@ hipError_t ioUpload(const IoHold&, hipStream_t stream, void* dst, const void* sr
 hipError_t ioDownload(const IoHold&, hipStream_t stream, void* dst, const void* src, size_t bytes)
 {
     if (bytes >= kIoDownloadLeast) {
+        const StreamDevice at(stream);
         Lease lease;
         const size_t per = ioChunk(bytes, 1, 4096);
         auto size = [&](size_t i) { return std::min(per, bytes - i * per); };
-        if (const SlotSet* set = lease.prepare())
+        if (const SlotSet* set = at.status == hipSuccess ? lease.prepare(at) : nullptr)
             return run(
                 *set, stream, (bytes + per - 1) / per, nullptr,
                 [&](size_t i, char* slot) { return hipMemcpyAsync(slot, static_cast<const char*>(src) + i * per, size(i), hipMemcpyDeviceToHost, stream); },

@@ -37,8 +37,9 @@ struct IoHold {
 // Where pinned memory is refused the chunks pass one after another through 3 MB
 // of device memory and of pageable memory instead.
 // fill and drain run in several threads and may be empty; enqueue, like every
-// call of the runtime, runs in the caller's thread, in order.  Returns when
-// every chunk is through; the first error ends it.
+// call of the runtime, runs in the caller's thread, in order, with the stream's
+// device as the current one.  Returns when every chunk is through; the first
+// error ends it.
 using IoEnqueue = std::function<hipError_t(size_t chunk, char* slot)>;
 using IoHost = std::function<void(size_t chunk, char* slot)>;
 hipError_t ioRun(const IoHold& hold, hipStream_t stream, size_t chunks, const IoHost& fill, const IoEnqueue& enqueue, const IoHost& drain);

@@ -1092,12 +1092,7 @@ int readScores(const dxg_world* w, bool want_e, bool want_e2, bool want_events, 
         split(slot, m, e, e2, ev);
         take(v, m, e, e2, ev);
     };
-    int before = 0;   // the caller's current device, put back below
-    HIP_TRY(hipGetDevice(&before));
-    HIP_TRY(hipSetDevice(w->device));
-    const hipError_t status = dxg::ioRun(w->io, w->stream, (n + per - 1) / per, nullptr, enqueue, drain);
-    HIP_TRY(hipSetDevice(before));
-    HIP_TRY(status);
+    HIP_TRY(dxg::ioRun(w->io, w->stream, (n + per - 1) / per, nullptr, enqueue, drain));
     return DXG_OK;
 }
 

@@ -237,6 +237,14 @@ int main(int argc, char** argv)
         CHECK(g_last_error == hipSuccess);   // the next launch check must not report it
         g_refuse_pinned = false;
         everything();
+    } else if (what == "stream of another device") {
+        everything();   // leaves a set with the events of device 0
+        g_stream.device = 1;
+        everything();
+        CHECK(g_current_device == 0);
+        g_current_device = 1;
+        everything();
+        CHECK(g_current_device == 1);
     } else if (what == "threads refused") {
         g_refuse_threads = true;
         everything();

@@ -1,6 +1,6 @@
 """Pinned-slot transfers (opendxmc_amd/csrc/hostio.cpp) on a stand-in for the
-HIP runtime that refuses pinned memory or threads: tests/cpp/hostio_check.cpp,
-one case a test."""
+HIP runtime: pinned memory or threads refused, other current devices.
+tests/cpp/hostio_check.cpp, one case a test."""
 from __future__ import annotations
 
 import subprocess
@@ -21,7 +21,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["plain", "pinned memory refused", "threads refused"])
+@pytest.mark.parametrize("case", ["plain", "pinned memory refused", "threads refused", "stream of another device"])
 def test_transfers(program, case):
     r = subprocess.run([str(program), case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -232,10 +232,8 @@ hipError_t run(const SlotSet& set, hipStream_t stream, size_t chunks, const IoHo
             if (e == hipSuccess) {
                 finished.store(f + 1, std::memory_order_release);
                 moved = true;
-            } else if (e != hipErrorNotReady) {
+            } else if (e != hipErrorNotReady) {   // not ready is not recorded as the last error
                 status = e;
-            } else {
-                (void)hipGetLastError();   // not ready is no error
             }
         }
         return moved;

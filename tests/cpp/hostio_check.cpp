@@ -245,6 +245,12 @@ int main(int argc, char** argv)
         g_current_device = 1;
         everything();
         CHECK(g_current_device == 1);
+    } else if (what == "earlier error") {   // stays for the caller to find, as after the runtime's own calls
+        g_last_error = hipErrorInvalidDevice;
+        g_lag = std::chrono::milliseconds(1);
+        dxg::IoHold hold;
+        transfer(hold, 5, true, true);
+        CHECK(g_last_error == hipErrorInvalidDevice);
     } else if (what == "threads refused") {
         g_refuse_threads = true;
         everything();

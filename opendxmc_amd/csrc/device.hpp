@@ -242,7 +242,7 @@ void launchBatchFinish(const DevParams* params, int n_inst, DevCounters* out, hi
 // The scores of voxels [0, n) of `tally` (records of kTallyRecord doubles) as
 // arrays: sum w dE and sum (w dE)^2 as doubles, the events as integers; each to
 // its array unless null.  The arrays may be device-accessible host memory.
-void launchScores(const double* tally, uint64_t n, double* sum_e, double* sum_e2, uint64_t* events, hipStream_t s);
+hipError_t launchScores(const double* tally, uint64_t n, double* sum_e, double* sum_e2, uint64_t* events, hipStream_t s);
 // Source particles of beam histories [0, n): 8 floats each (ax, ay, direction,
 // E, w, exposure index), from the transport kernels' sampling code.
 void launchSource(const DevParams& p, uint64_t n, float* out, hipStream_t s);

@@ -1547,11 +1547,13 @@ void launchBatchFinish(const DevParams* params, int n_inst, DevCounters* out, hi
     hipLaunchKernelGGL(batch_finish_kernel, dim3(parts * static_cast<unsigned>(n_inst)), dim3(256), 0, s, params, parts, out);
 }
 
-void launchScores(const double* tally, uint64_t n, double* sum_e, double* sum_e2, uint64_t* events, hipStream_t s)
+hipError_t launchScores(const double* tally, uint64_t n, double* sum_e, double* sum_e2, uint64_t* events, hipStream_t s)
 {
     if (n == 0)
-        return;
-    hipLaunchKernelGGL(scores_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s, tally, n, sum_e, sum_e2, events);
+        return hipSuccess;
+    // the launch's own status: the thread's last error may be an earlier call's
+    void* args[] = { &tally, &n, &sum_e, &sum_e2, &events };
+    return hipLaunchKernel(reinterpret_cast<const void*>(scores_kernel), dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), args, 0, s);
 }
 
 void launchReset(unsigned long long* pool, DevCounters* counters, hipStream_t s)

@@ -1082,8 +1082,7 @@ int readScores(const dxg_world* w, bool want_e, bool want_e2, bool want_events, 
         double *e, *e2;
         uint64_t* ev;
         split(slot, m, e, e2, ev);
-        dxg::launchScores(w->d_tally.ptr + v * dxg::kTallyRecord, m, e, e2, ev, w->stream);
-        return hipGetLastError();
+        return dxg::launchScores(w->d_tally.ptr + v * dxg::kTallyRecord, m, e, e2, ev, w->stream);
     };
     auto drain = [&](size_t c, char* slot) {
         const uint64_t v = c * per, m = std::min(per, n - v);

@@ -17,7 +17,7 @@ from opendxmc_amd import _native as N
 from opendxmc_amd import build
 from opendxmc_amd import phantoms
 from opendxmc_amd import pipelines as P
-from opendxmc_amd.devmem import DeviceBuffer
+from opendxmc_amd.devmem import DeviceBuffer, _rt
 from physics_refs import MGY_PER_KEV_G
 
 pytestmark = pytest.mark.gpu
@@ -67,6 +67,21 @@ def test_scores_read_whole(dims):
         N.check(N.lib().dxg_read_energy_scores(grid._h, *[p if i == k else None for i, p in enumerate(ptrs)]))
         np.testing.assert_array_equal(out[k], (e, e2, ev)[k])
         assert all((out[i] == 7).all() for i in range(3) if i != k)
+
+
+@pytest.mark.parametrize("dims", [(16, 16, 16), (101, 97, 43)])
+def test_read_after_an_unrelated_error(dims):
+    """An error that an earlier call of the runtime left behind on the thread is
+    not taken for the read's own."""
+    _, grid, _ = scored_world(dims)
+    want = grid.doseScored()
+    assert _rt().hipSetDevice(9999) != 0
+    try:
+        for a, b in zip(grid.doseScored(), want):
+            np.testing.assert_array_equal(a, b)
+        assert _rt().hipPeekAtLastError() != 0      # still its owner's to find
+    finally:
+        _rt().hipGetLastError()
 
 
 def test_concurrent_reads():

@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstring>
 #include <exception>
 #include <memory>
@@ -186,12 +187,24 @@ hipError_t run(const SlotSet& set, hipStream_t stream, size_t chunks, const IoHo
     auto vacant = [&](size_t c) {
         return c < kIoSlots || (drain ? drained[at(c)].load(std::memory_order_acquire) == c - kIoSlots + 1 : arrived(c - kIoSlots));
     };
+    // A wait between chunks is short (3 MB take 57 us of the link); one for work
+    // enqueued before, many layers of a network, say, must not keep every worker's
+    // CPU busy.
     auto wait = [&](auto ready) {
+        using Clock = std::chrono::steady_clock;
+        Clock::time_point start;
         for (size_t spin = 0; !ready(); ++spin) {
             if (stop.load(std::memory_order_relaxed))
                 return false;
-            if (spin > 64)
+            if (spin <= 64)
+                continue;
+            if (spin == 65)
+                start = Clock::now();
+            const Clock::duration waited = Clock::now() - start;
+            if (waited < std::chrono::milliseconds(1))
                 std::this_thread::yield();
+            else
+                std::this_thread::sleep_for(waited / 64);   // at most 1.6 % late
         }
         return true;
     };

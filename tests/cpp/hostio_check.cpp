@@ -251,6 +251,14 @@ int main(int argc, char** argv)
         dxg::IoHold hold;
         transfer(hold, 5, true, true);
         CHECK(g_last_error == hipErrorInvalidDevice);
+    } else if (what == "waiting") {   // on device work of 0.4 s: at most the caller keeps a CPU busy
+        g_lag = std::chrono::milliseconds(400);
+        dxg::IoHold hold;
+        const std::clock_t before = std::clock();   // CPU time of all threads
+        transfer(hold, 2 * dxg::kIoThreads, false, true);
+        const double busy = static_cast<double>(std::clock() - before) / CLOCKS_PER_SEC;
+        std::printf("%.2f s of CPU time\n", busy);
+        CHECK(busy < 1.2);   // two waits (16 slots): 0.8 s of the caller
     } else if (what == "threads refused") {
         g_refuse_threads = true;
         everything();

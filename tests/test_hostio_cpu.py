@@ -21,7 +21,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["plain", "pinned memory refused", "threads refused", "stream of another device", "earlier error"])
+@pytest.mark.parametrize("case", ["plain", "pinned memory refused", "threads refused", "stream of another device", "earlier error", "waiting"])
 def test_transfers(program, case):
     r = subprocess.run([str(program), case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr

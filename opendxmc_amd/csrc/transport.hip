@@ -12,9 +12,9 @@
 // Each loop iteration a wavefront runs exactly ONE phase, chosen from ballots
 // of the lane states, with the lanes of the other states masked off:
 //   * refill   once refill_threshold lanes are DEAD (or nothing else can run):
-//              they take consecutive ids from the wavefront's private batch of
-//              pool histories (one global atomic per `batch` histories) and
-//              sample their source particle together;
+//              they take photons from the work-group's source queue, which one
+//              of its wavefronts at a time fills with 64 histories of the
+//              group's claim (one global atomic per `batch` histories);
 //   * interact once interact_threshold lanes are parked (or no lane tracks
 //              and fewer than outer_threshold wait for outer flights):
 //              photoelectric / Compton / Rayleigh for all parked lanes at

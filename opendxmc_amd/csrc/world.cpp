@@ -838,7 +838,7 @@ int worldDevice(const dxg_world* w) { return w->device; }
 // Launch settings chosen by the run's own timing, kept per world build and
 // beam layout: dead lanes that start a refill, parked lanes that start an
 // interaction phase, lanes outside the box that start an outer-flight phase,
-// and histories a wavefront claims per pool atomic.  Events, tallies and
+// and histories a work-group claims per pool atomic, at most.  Events, tallies and
 // scores do not depend on them (per-history random streams), only time does.
 struct Tuned {
     int refill, interact, outer;
@@ -917,6 +917,7 @@ int runChunks(dxg_world* w, DevParams& p, uint64_t total, dxg_progress* progress
     dxg_counters acc {};
     int status = DXG_OK;
     const bool explicit_batch = std::getenv("DXG_BATCH") != nullptr;
+    acc.batch = p.batch;
     // one launch over beam histories [h_begin, h_end); ms receives its time
     auto launchRange = [&](uint64_t h_begin, uint64_t h_end, float& ms) -> int {
         p.h_begin = h_begin;
@@ -924,6 +925,7 @@ int runChunks(dxg_world* w, DevParams& p, uint64_t total, dxg_progress* progress
         const unsigned long long most = p.batch;   // put back below: later ranges may be longer
         if (!explicit_batch)
             p.batch = dxg::claimSize(h_end - h_begin, blocks, most);
+        acc.batch = p.batch;
         const auto turn = w->turns.change();   // until the histories are counted
         dxg::launchReset(p.pool, p.counters, w->stream);
         const auto t0 = std::chrono::steady_clock::now();
@@ -1044,7 +1046,6 @@ int runChunks(dxg_world* w, DevParams& p, uint64_t total, dxg_progress* progress
     acc.refill_threshold = p.refill_threshold;
     acc.interact_threshold = p.interact_threshold;
     acc.outer_threshold = p.outer_threshold;
-    acc.batch = p.batch;
     acc.autotuned = autotuned;
     w->counters = acc;
     if (progress && status == DXG_OK)

@@ -447,6 +447,20 @@ def test_autotuned_launch_settings_leave_results_unchanged():
     assert counts["tuned"] == counts["default"]
 
 
+@pytest.mark.parametrize("histories,explicit,claim", [(1000, None, 64), (1000, "128", 128), (100_000_000, None, 512)])
+def test_counters_report_the_claim_of_the_run(histories, explicit, claim, monkeypatch):
+    """A run too short for every work-group's full claim takes smaller ones, and
+    says so; an explicit claim is taken as given."""
+    monkeypatch.setenv("DXG_AUTOTUNE", "0")
+    if explicit:
+        monkeypatch.setenv("DXG_BATCH", explicit)
+    world, grid = make_world(phantoms.water_cube(16, 0.2), 0)
+    beam = dx.PencilBeam((0.1, 0.1, -10.0), (0.0, 0.0, 1.0), 60.0)
+    beam.setNumberOfParticlesPerExposure(histories)
+    assert dx.Transport(seed=5)(world, beam, None, False)
+    assert grid.counters()["batch"] == claim
+
+
 def test_air_fill_medium_effect_on_the_pencil_cube():
     """The world here ends at the grid (vacuum beyond); DXMClib's World fills
     the space around its items with air (its padding is not in the reference

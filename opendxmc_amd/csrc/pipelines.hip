@@ -689,9 +689,11 @@ int dxg_ct_segment(const dxg_ct_segmentation* t, const double* hu, uint64_t n, u
         return DXG_OK;
     if (!hu || !material || !density)
         return fail(DXG_ERR_ARGUMENT, "dxg_ct_segment: null argument");
-    // through slots, except that small volumes gain nothing by it and that outputs
-    // over the input may be written only after all of it was read
-    if (n >= kSegHostLeast && !overlap(hu, n * sizeof(double), material, n) && !overlap(hu, n * sizeof(double), density, n * sizeof(double)))
+    // through slots, except that small volumes gain nothing by it, that outputs
+    // over the input may be written only after all of it was read, and that of
+    // outputs over each other the densities, written last, are to stay whole
+    if (n >= kSegHostLeast && !overlap(hu, n * sizeof(double), material, n) && !overlap(hu, n * sizeof(double), density, n * sizeof(double))
+        && !overlap(material, n, density, n * sizeof(double)))
         return segmentHost(*t, hu, n, material, density);
     DeviceBuffer<double> dh, dd;
     DeviceBuffer<uint8_t> dm;

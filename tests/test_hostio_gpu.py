@@ -131,7 +131,7 @@ def test_read_during_runs_is_a_state_between_launches():
 def test_segmentation_of_host_arrays_equals_resident(n):
     """The same bits whichever way the voxels travel, below 393,216 voxels through
     whole device buffers and from there in chunks; with the densities over the CT
-    numbers too."""
+    numbers too, and over the materials."""
     rng = np.random.default_rng(n)
     hu = rng.uniform(-1100.0, 2500.0, n)
     hu[rng.integers(0, n, 5)] = [np.nan, np.inf, -np.inf, -0.0, -1000.0]
@@ -145,6 +145,9 @@ def test_segmentation_of_host_arrays_equals_resident(n):
     over = hu.copy()
     N.check(N.lib().dxg_ct_segment(C.byref(tables), N.ptr(over, C.c_double), n, N.ptr(m, C.c_uint8), N.ptr(over, C.c_double)))
     np.testing.assert_array_equal(over.view(np.uint64), dens.view(np.uint64))
+    # the materials over the densities: those are written last
+    N.check(N.lib().dxg_ct_segment(C.byref(tables), N.ptr(hu, C.c_double), n, N.ptr(d.view(np.uint8), C.c_uint8), N.ptr(d, C.c_double)))
+    np.testing.assert_array_equal(d.view(np.uint64), dens.view(np.uint64))
     assert P.last_ms(0) > 0.0
 
 

@@ -227,27 +227,17 @@ struct RowsTile {
 // bit 1 row y + 1 (a pair index counts (n, z, y / 2, x / 64) like a tile
 // index with ceil(ny / 2) rows); without a list every pair is computed and
 // row y + 1 is stored when it exists.
-// The epilogue's configuration as template bits (EPI >= 0), so that a layer's
-// code holds only its own epilogue: the runtime tests of the residual, gate,
-// activation and output kind cost instructions (and branches) on every store.
-// EPI < 0 reads the configuration from the arguments.
+// The epilogue's configuration as template bits, so that a layer's code holds
+// only its own epilogue: run-time tests of the residual, gate, activation and
+// output kind cost instructions (and branches) on every store.
 constexpr int kEpiRelu = 1, kEpiRes = 2, kEpiGate = 4, kEpiY = 8, kEpiY32 = 16, kEpiY32All = 32;
-
-template <int EPI>
-__device__ inline bool epiHas(int flag, bool runtime)
-{
-    return EPI < 0 ? runtime : (EPI & flag) != 0;
-}
 
 template <int R, int EPI>
 __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu(kConvWaves / 2))) void conv3d_rows_kernel(ConvArgs a)
 {
-    const bool e_relu = epiHas<EPI>(kEpiRelu, a.relu != 0);
-    const bool e_res = epiHas<EPI>(kEpiRes, a.res != nullptr);
-    const bool e_gate = epiHas<EPI>(kEpiGate, a.gate != nullptr);
-    const bool e_y = epiHas<EPI>(kEpiY, a.y != nullptr);
-    const bool e_y32 = epiHas<EPI>(kEpiY32 | kEpiY32All, a.y32 != nullptr);
-    const bool e_y32_all = epiHas<EPI>(kEpiY32All, a.y32_channels == kC);
+    static_assert(R <= 2 && kConvWaves <= 4, "the residual and gate values of more rows leave no registers for the ring");
+    constexpr bool e_relu = EPI & kEpiRelu, e_res = EPI & kEpiRes, e_gate = EPI & kEpiGate, e_y = EPI & kEpiY;
+    constexpr bool e_y32_all = EPI & kEpiY32All, e_y32 = e_y32_all || (EPI & kEpiY32);
     // the single-channel FP32 output (the last layer) needs output channels
     // 0-15 only: the second channel half's MFMAs and weight reads are skipped
     constexpr int kHalves = EPI == kEpiY32 ? 1 : 2;
@@ -386,10 +376,7 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
         // epilogue waited on each other (input gradients of a training step on
         // 4 x 64^3 voxels: 3.54 ms of device time a step, so 3.49)
         const size_t orow0 = (static_cast<size_t>(n * a.nz + z) * a.ny + y) * a.nx;
-        // (up to two rows: more would not leave registers for the ring)
-        constexpr bool kPrefetchSide = R <= 2 && kConvWaves <= 4;
-        u32x2 side[kPrefetchSide ? R : 1][4][2];
-        const uint16_t* side_src = e_res ? a.res : (e_gate ? a.gate : nullptr);
+        u32x2 side[R][4][2];
         auto loadSide = [&](const uint16_t* from) {
 #pragma unroll
             for (int o = 0; o < R; ++o) {
@@ -399,12 +386,12 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
                 for (int j = 0; j < 4; ++j)
 #pragma unroll
                     for (int m = 0; m < 2; ++m)
-                        side[kPrefetchSide ? o : 0][j][m] = *reinterpret_cast<const u32x2*>(
+                        side[o][j][m] = *reinterpret_cast<const u32x2*>(
                             from + (orow0 + static_cast<size_t>(o) * a.nx + x0) * kC + out_off + j * kPhase + m * 2 * kChunk);
             }
         };
         uint32_t open[R] = {};   // with both: which outputs the gate lets through
-        if (kPrefetchSide && (e_res || e_gate))
+        if (e_res || e_gate)
             loadSide(e_gate ? a.gate : a.res);
 
 #pragma unroll
@@ -414,14 +401,14 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
                 loadRow(cur, q + kAhead, (q + kAhead) % kRing);
             else
                 loadRow(nxt, q + kAhead - kRows, (q + kAhead) % kRing);
-            if (kPrefetchSide && e_res && e_gate && q == 2) {
+            if (e_res && e_gate && q == 2) {
 #pragma unroll
                 for (int o = 0; o < R; ++o)
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
 #pragma unroll
                         for (int m = 0; m < 2; ++m) {
-                            const u32x2 gv = side[kPrefetchSide ? o : 0][j][m];
+                            const u32x2 gv = side[o][j][m];
                             const uint32_t h[4] = { gv[0] << 16, gv[0] & 0xffff0000u, gv[1] << 16, gv[1] & 0xffff0000u };
                             for (int i = 0; i < 4; ++i)
                                 open[o] |= static_cast<int>(h[i]) > 0 ? 1u << (j * 8 + m * 4 + i) : 0u;
@@ -489,10 +476,8 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
                     float out[4];
                     for (int i = 0; i < 4; ++i)
                         out[i] = acc[o][m][j][i] + bias[m][i];
-                    const u32x2 sv = kPrefetchSide ? side[kPrefetchSide ? o : 0][j][m]
-                                                   : ((e_res || e_gate) ? *reinterpret_cast<const u32x2*>(side_src + at) : u32x2 { 0, 0 });
                     if (e_res) {
-                        const u32x2 rv = sv;
+                        const u32x2 rv = side[o][j][m];
                         out[0] += fromBf16(rv[0] & 0xffffu);
                         out[1] += fromBf16(rv[0] >> 16);
                         out[2] += fromBf16(rv[1] & 0xffffu);
@@ -501,12 +486,12 @@ __global__ __launch_bounds__(64 * kConvWaves) __attribute__((amdgpu_waves_per_eu
                     if (e_relu)
                         for (int i = 0; i < 4; ++i)
                             out[i] = fmaxf(out[i], 0.0f);
-                    if (kPrefetchSide && e_res && e_gate) {
+                    if (e_res && e_gate) {
                         for (int i = 0; i < 4; ++i)
                             if (!((open[o] >> (j * 8 + m * 4 + i)) & 1))
                                 out[i] = 0.0f;
                     } else if (e_gate) {
-                        const u32x2 gv = e_res ? *reinterpret_cast<const u32x2*>(a.gate + at) : sv;
+                        const u32x2 gv = side[o][j][m];
                         const uint32_t h[4] = { gv[0] & 0xffffu, gv[0] >> 16, gv[1] & 0xffffu, gv[1] >> 16 };
                         for (int i = 0; i < 4; ++i)
                             if (h[i] == 0 || (h[i] & 0x8000u))
@@ -672,8 +657,8 @@ __global__ __launch_bounds__(64 * kConvWaves) void conv3d_first_kernel(ConvArgs 
     }
 }
 
-// The row kernel for a launch's epilogue: the configurations the network and
-// the probe use are compiled on their own; any other reads its flags at run time.
+// The row kernel for a launch's epilogue, one of the configurations that the
+// network and the probe use; null for any other.
 const void* rowsKernel(const ConvArgs& a)
 {
     const int epi = (a.relu ? kEpiRelu : 0) | (a.res ? kEpiRes : 0) | (a.gate ? kEpiGate : 0) | (a.y ? kEpiY : 0)
@@ -692,7 +677,7 @@ const void* rowsKernel(const ConvArgs& a)
     case kEpiY32All:
         return reinterpret_cast<const void*>(&conv3d_rows_kernel<kConvRows, kEpiY32All>);
     default:
-        return reinterpret_cast<const void*>(&conv3d_rows_kernel<kConvRows, -1>);
+        return nullptr;
     }
 }
 
@@ -1248,8 +1233,8 @@ struct Dims {
     size_t voxels() const { return static_cast<size_t>(nb) * nz * ny * nx; }
 };
 
-// Whether the first layer runs conv3d_first_kernel on the compact input: row
-// pairs on, and a plane small enough for its 32-bit offsets.
+// Whether the first layer runs conv3d_first_kernel on the compact input: a plane
+// small enough for its 32-bit offsets.
 bool firstLayerCompact(const Dims& d)
 {
     return convFirst() && static_cast<long long>(d.ny + 1) * d.nx < (1ll << 27);
@@ -1310,8 +1295,11 @@ hipError_t launchConv(ConvArgs a, const Dims& d, hipStream_t s)
             return hipErrorInvalidValue;
         hipLaunchKernelGGL(conv3d_first_kernel, dim3(grid), dim3(64 * kConvWaves), 0, s, a);
     } else {
+        const void* const kernel = rowsKernel(a);
+        if (!kernel)
+            return hipErrorInvalidValue;
         void* args[] = { &a };
-        (void)hipLaunchKernel(rowsKernel(a), dim3(grid), dim3(64 * kConvWaves), args, 0, s);
+        (void)hipLaunchKernel(kernel, dim3(grid), dim3(64 * kConvWaves), args, 0, s);
     }
     return hipGetLastError();
 }

@@ -11,12 +11,14 @@ restatement, and that training lowers the loss.
 from __future__ import annotations
 
 import ctypes as C
+import subprocess
 
 import numpy as np
 import pytest
 import torch
 
 from opendxmc_amd import _native as N
+from opendxmc_amd import build
 from opendxmc_amd import denoise as dn
 from opendxmc_amd.devmem import _rt
 
@@ -48,6 +50,16 @@ def test_parameter_count():
     # the unpadded network: 4->32, 16 x 32->32, 32->1
     live = (4 * 27 * 32 + 32) + 16 * (32 * 27 * 32 + 32) + (32 * 27 + 1)
     assert live == 447_233
+
+
+def test_initial_weights_draw_as_the_standard_library(tmp_path):
+    """The initial weights of a seed are those that std::normal_distribution<float>
+    of this image's standard library gives."""
+    exe = tmp_path / "normals_check"
+    subprocess.run(["g++", "-std=c++17", "-O2", f"-I{build.CSRC}", str(build.TESTS_CPP / "normals_check.cpp"), "-o", str(exe)],
+                   check=True, timeout=120)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
 
 
 def test_probe_rejects_bad_shapes():

@@ -324,6 +324,34 @@ def test_network_loss_and_gradients_match_reference():
             assert np.all(g[:ref.LAYER_W].reshape(32, 27, 32)[1:] == 0) and np.all(g[ref.LAYER_W + 1:] == 0)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,dims", [(1, (3, 4, 128)), (2, (2, 8, 192)), (1, (1, 4, 64)), (1, (9, 36, 128))])
+def test_gradients_across_x_tiles(batch, dims):
+    """Every layer's gradient where x tiles have neighbours and row ranges cross
+    tiles, planes and volumes: the weight gradient of the first layer (one live
+    half of the input channels) and of the last (one live half of the output
+    channels), and the input gradients with residual and gate.  Two evaluations
+    that round to BF16 and sum in different orders lie about equally far from the
+    exact gradient: the largest deviation may be twice the restatement's own
+    (0.003 .. 0.02 of the largest value for the larger volumes, 0.005 .. 0.08 for
+    256 voxels), the mean one as in the test above."""
+    params = ref.random_params(33, scale=0.8)
+    net = dn.Denoiser(seed=1)
+    net.set_params(params)
+    f, target, mask = _net_case(34, batch, dims)
+    net.train_step(f, target, mask, lr=1e-6)
+    grads = net.grads().astype(np.float64)
+    _, _, rgrads = ref.loss_and_grads(params, f, target, mask)
+    _, _, egrads = ref.loss_and_grads(params, f.astype(np.float64), target.astype(np.float64),
+                                      mask.astype(np.float64), rounding=False, dtype=torch.float64)
+    for l in range(ref.LAYERS):
+        g, r, e = (a[l * ref.LAYER_P:(l + 1) * ref.LAYER_P] for a in (grads, rgrads, egrads))
+        scale = np.abs(e).max()
+        dev, noise = _rounding_noise(g, r, e)
+        assert dev <= 2.0 * noise + 1e-5 * scale, l
+        assert np.abs(g - e).max() <= 2.0 * np.abs(r - e).max(), l
+
+
 def _free_memory() -> int:
     free, total = C.c_size_t(), C.c_size_t()
     assert _rt().hipMemGetInfo(C.byref(free), C.byref(total)) == 0

@@ -220,8 +220,11 @@ struct DevParams {
 // 512: 0.8); kernel ms of a 64^3 pencil beam at 1e6 / a 97x161x79 DX field at
 // 5e6 / the 512x512x64 dual-source slab at 3e7 / the 256x256x200 spiral at 1e8:
 // 256 0.136 / 0.69 / 2.68 / 9.23, 512 0.121 / 0.65 / 2.63 / 9.17, 1024 0.139 /
-// 0.65 / 2.66 / 9.18, 2048 0.180 / 0.67 / 2.68 / 9.19.  Never more than the
-// work-group's share, so that a small run reaches every work-group.
+// 0.65 / 2.66 / 9.18, 2048 0.180 / 0.67 / 2.68 / 9.19.  Whole calls with 64 / 256
+// / 512 / 1024 on a 1 cm field into 48^3 at 1e7: 2.32 / 1.20 / 1.12 / 1.15, two
+// slices of 80^3 at 5e6 1.20 / 0.50 / 0.46 / 0.46 and of a 128x128x90 body at 2e7
+// 4.39 / 1.79 / 1.77 / 1.77.  Never more than the work-group's share, so that a
+// small run reaches every work-group.
 inline unsigned long long claimSize(unsigned long long histories, int blocks, unsigned long long most = 512)
 {
     const unsigned long long share = histories / static_cast<unsigned long long>(blocks) / 64 * 64;

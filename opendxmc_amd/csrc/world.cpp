@@ -526,7 +526,11 @@ int dxg_world_build(dxg_world* w)
     // and a fold after each run sums them.  Up to 8 copies within 128 MiB: a
     // call with a pencil beam into 64^3 water took, with 1 / 2 / 4 / 8 / 16
     // copies, 0.40 / 0.25 / 0.228 / 0.225 / 0.235 ms at 1e6 histories and 25.9 /
-    // 9.1 / 6.25 / 5.99 / 6.41 ms at 1e8 (16 copies fall out of the caches).
+    // 9.1 / 6.25 / 5.99 / 6.41 ms at 1e8 (16 copies fall out of the caches).  With
+    // 1 / 4 / 8 / 16 copies: a pencil into 32^3 at 2e7 10.9 / 1.85 / 1.32 / 1.31, a
+    // 1 cm field on 48^3 at 1e7 1.71 / 1.22 / 1.17 / 1.17, fields over the whole
+    // object on 64x96x40 at 2e6 0.448 / 0.466 / 0.477 / 0.498 and on 128x128x90 at
+    // 2e7 1.77 / 1.79 / 1.87 / 2.08: what a wide field loses is small.
     {
         const size_t bytes = w->tallyDoubles() * sizeof(double);
         w->replicas = static_cast<int>(std::clamp<size_t>((size_t(128) << 20) / std::max<size_t>(bytes, 1), 1, 8));

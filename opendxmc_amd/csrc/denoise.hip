@@ -1940,6 +1940,16 @@ size_t valueAt(size_t i)
     return chunkAt(v & ~static_cast<size_t>(63), static_cast<int>(v & 63), c >> 3) + (c & 7);
 }
 
+// In a function of its own: inlined into a long one, the sum was kept in memory
+// from addition to addition (0.3 ms more on 4 x 64^3 voxels).
+__attribute__((noinline)) double maskSum(const float* mask, size_t n)
+{
+    double sum = 0.0;
+    for (size_t i = 0; i < n; ++i)
+        sum += mask[i];
+    return sum;
+}
+
 bool hasDevice()
 {
     int n = 0;
@@ -2077,9 +2087,7 @@ int dxg_denoiser_train_step(dxg_denoiser* d, const float* features, const float*
         return rc;
     if (int rc = d->toDevice(d->mask.p, mask, nv * sizeof(float), d->copies); rc != DXG_OK)
         return rc;
-    double count = 0.0;
-    for (size_t i = 0; i < nv; ++i)
-        count += mask[i];
+    const double count = maskSum(mask, nv);
     if (!(count > 0.0))
         return fail(DXG_ERR_ARGUMENT, "dxg_denoiser_train_step: empty mask");
     HIP_TRY(d->gbuf.reserve(3 * nv * kC));

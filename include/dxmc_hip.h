@@ -189,7 +189,9 @@ int dxg_transport_run_static(dxg_world* w, const dxg_beam* beam, dxg_progress* p
 /* Zero the energy scores and the history count. */
 int dxg_world_clear_scores(dxg_world* w);
 
-/* EnergyScore per voxel: sum of w*dE (keV), sum of (w*dE)^2 (keV^2), events. */
+/* EnergyScore per voxel: sum of w*dE (keV), sum of (w*dE)^2 (keV^2), events.
+ * While another thread runs the world with dxg_transport_run, a read gives the
+ * scores between two launches of the run.  Any output pointer may be null. */
 int dxg_read_energy_scores(const dxg_world* w, double* sum_e, double* sum_e2, uint64_t* n_events);
 
 /* DoseScore per voxel: vgrid.doseScored(i).{dose(), variance(), numberOfEvents()}

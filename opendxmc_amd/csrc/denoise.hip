@@ -106,8 +106,11 @@ __device__ inline u32x4 load16(const uint16_t* p) { return *reinterpret_cast<con
 // With a voxel's 32 channels contiguous instead, each 16-lane pass of a load
 // fell in 16 cache lines and the texture address units were 95 % busy: 18
 // layers of 128x256x256 voxels 11.1 ms, so 8.4 (8.2 with the weights straight to
-// LDS: 985 TFLOP/s a full layer, where a library product of 8192^3 reaches 1157;
-// both hold the clock at 1.5-1.9 of 2.4 GHz, so power bounds them).
+// LDS: 985 TFLOP/s a full layer).  What bounds a full layer of that volume now is
+// the clock, which falls from 2.4 to 1.57-1.86 GHz (a library product of 8192^3
+// runs at 1.84-1.92 GHz and 1334-1400 TFLOP/s), together with 4.9-6.1 TB/s of
+// traffic past L2 and texture data units that are 90 % busy; layers of 4 x 64^3
+// voxels run at 2.2-2.5 GHz.
 constexpr int kTile = 64 * kC;          // values of a tile
 constexpr int kPhase = 16 * kC;         // ... of a phase
 constexpr int kChunk = 16 * 8;          // ... of a phase's channel chunk
@@ -696,7 +699,9 @@ struct WgradArgs {
 // channels] with voxel n of a phase in slot n + 1; slot 0 of phase 3 holds the
 // voxel before the row and slot 17 of phase 0 the one after.  A chunk takes 320
 // bytes: the two chunks and four voxels that a 16-lane group of a transposing
-// read covers then fall in distinct banks.
+// read covers then fall in distinct banks.  Neighbouring groups still share half
+// of theirs (chunk 1 of one and chunk 0 of the next), and the four phases start in
+// one bank, which the halo write meets: conflicts take 35 % of the LDS cycles.
 constexpr int kWgChunk = 320, kWgPhase = 4 * kWgChunk, kWgRow = 4 * kWgPhase;
 constexpr int kWgWaves = 4;
 constexpr int kWgPart = 9 * 32 * 32;   // values of a work-group's partial sums
@@ -725,8 +730,10 @@ __device__ inline bf16x8 joinOperand(s16x4 lo, s16x4 hi)
 // One layer on 4 x 64^3 voxels (58 GFLOP): 63 us, 920 TFLOP/s (73 us with the
 // compiler's own order of a step's instructions); a kernel that transposed rows
 // by two-byte LDS writes and read them back for each tap took 196 us, bound by
-// LDS.  What bounds it now: the matrix pipes and, as the variants with half of
-// the products still take 51 and 55 us, the three passes over x and g.
+// LDS.  What bounds it now is no one unit: at 2.5 GHz the matrix pipes are busy
+// 39 % of the time, a wavefront waits 30 % of its cycles to issue and 25 % for
+// loads and LDS (with its bank conflicts), with no second wavefront on the SIMD to
+// fill them; the variants with half of the products still take 51 and 55 us.
 template <int CO, int CI>
 __global__ __launch_bounds__(64 * kWgWaves) __attribute__((amdgpu_waves_per_eu(1, 1))) void wgrad_kernel(WgradArgs a)
 {
@@ -2056,6 +2063,7 @@ int dxg_denoiser_train_step(dxg_denoiser* d, const float* features, const float*
     Dims dm {};
     if (int rc = checkDims("dxg_denoiser_train_step", batch, dims, dm); rc != DXG_OK)
         return rc;
+    // (a limit of the interface: the kernels take any y extent)
     if (dm.ny % 4 != 0)
         return fail(DXG_ERR_ARGUMENT, "dxg_denoiser_train_step: the y extent must be a multiple of 4");
     if (!(lr > 0.0f) || !std::isfinite(lr))
